@@ -189,3 +189,62 @@ def test_room_image_converges_near_path_tracing(gpu_ctx, ilm, variant):
     sc.close()
     m.close()
     acc.free()
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("count", [31, 32, 33, 64, 65, 129])
+def test_lookups_at_list_lengths_around_the_masks(gpu_ctx, ilm, variant, count):
+    """Lists just short of and past the length that gets cell masks, whole and
+    part words, at thresholds below and above 1, with record normals and
+    lookup normals longer than 1 (which reach further). The whole lists in 64
+    bits give the sums; a weight w = 1 / x - 1 / threshold, x = d / RiClamp +
+    1 - cos, is off by x's rounding (a few 2^-24 of its terms, each at most
+    4 here) over x squared, plus its own, and a list's sum by its length
+    times 2^-24."""
+    m, sc, pos = _room(ilm, gpu_ctx)
+    rng = np.random.default_rng(count)
+    for threshold, scale in ((0.05, 1.0), (0.3, 1.0), (0.3, 1.5), (3.0, 1.0)):
+        ic = ilm.IrradianceCache(sc, cache_depth=1, error_threshold=threshold, ambient_resolution=0.01,
+                                 ambient_multiplier=10.0, variant=variant)
+        # cache depth 1: every record lies in the lists of the root's children
+        P = rng.random((count, 3)) * 0.4 + 0.05
+        N = np.array([0, 1, 0]) + 0.1 * rng.normal(size=(count, 3))
+        N *= scale / np.linalg.norm(N, axis=1, keepdims=True)
+        R = np.concatenate([P, N, rng.random((count, 3)), 0.1 + 0.2 * rng.random((count, 1))], 1).astype(np.float32)
+        ic.insert(R)
+        lists = [ic.node(k)[1] for k in range(ic.info()["nodes"])]
+        lo, hi = ic.info()["root"][:3], ic.info()["root"][3:]
+        centre = lo + (hi - lo) * np.float32(0.5)
+        q = 300
+        qn = np.tile(np.array([0, 1.0, 0]), (q, 1))
+        qn[::3] *= 2.0                             # beyond unit length: the whole list is walked
+        Q = np.concatenate([rng.random((q, 3)) * 0.5, qn], 1).astype(np.float32)
+        got = ic.lookup(Q).astype(np.float64)
+        rc, Rd, Qd, inv = ic.records()[:, 10].astype(np.float64), R.astype(np.float64), Q.astype(np.float64), \
+            float(np.float32(1) / np.float32(threshold))
+        assert max(len(x) for x in lists) == count
+        weighted = 0
+        for i in range(q):
+            b = Q[i, :3] > centre
+            r = lists[1 + int(b[0]) + 2 * int(b[2]) + 4 * int(b[1])]
+            d = np.linalg.norm(Rd[r, :3] - Qd[i, :3], axis=1) / rc[r]
+            cos = Rd[r, 3:6] @ Qd[i, 3:]
+            if variant == 0:
+                x = d + 1 - cos
+                w = np.where(cos > 0, 1 / x - inv, -1.0)
+                off = 24 * 2.0 ** -24 / x ** 2 + 4 * 2.0 ** -24 * (np.abs(1 / x) + inv)
+            else:
+                w = 1 - inv * np.maximum(d, (1 - cos) * 9.0124)
+                off = np.full(len(r), 48 * 2.0 ** -24 * (1 + inv))
+            w0 = np.where(w > 0, w, 0)
+            den = w0.sum()
+            bound = off[w > -off].sum() + len(r) * 2.0 ** -23 * den
+            assert abs(got[i, 3] - den) <= bound, (i, got[i, 3], den, bound)
+            if den > 100 * bound:
+                e = (w0[:, None] * Rd[r, 6:9]).sum(0) / den
+                assert np.abs(got[i, :3] - e).max() <= 2 * bound / den + len(r) * 2.0 ** -23
+                weighted += 1
+        assert weighted > 20 or threshold < 0.1
+        ic.close()
+    sc.close()
+    m.close()
