@@ -5,13 +5,12 @@
 // Replaces the host BVHMesh::Compile (Shape/BVHMesh.cpp:78-107,203-269) where
 // build time matters more than tree quality (many or large scenes).
 //
-// Steps (one stream, no host round trips except the per-level counts of the
-// collapse):
-//   1. triangle boxes; centroid bounds by block reduction + ordered-int atomics
+// Steps (one stream; the host waits once per batch of collapse levels):
+//   1. triangle boxes; centroid bounds by block reductions
 //   2. Morton codes (21 bits per axis) and radix sort of (code, triangle)
-//   3. Karras hierarchy: n-1 internal nodes, n leaves, parents and ranges
-//   4. refit: each leaf climbs; the second child to arrive unites the boxes
-//      (agent-scope acquire/release on the arrival counter)
+//   3. unions of the sorted leaf boxes over aligned runs of 2, 4, 8, ... leaves
+//   4. Karras hierarchy: n-1 internal nodes, n leaves; a node's box is the
+//      union of the runs its range of leaves is made of
 //   5. collapse, level by level: each wide node opens its largest-area
 //      internal children until it has four; a subtree of at most max_leaf
 //      triangles becomes one leaf (its triangles are contiguous in Morton order)
@@ -36,48 +35,63 @@ struct Box6 {
     float lo[3], hi[3];
 };
 
-__device__ __forceinline__ uint32_t ordered(float f) {
-    uint32_t u = __float_as_uint(f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+__device__ __forceinline__ Box6 empty_box() {
+    return Box6{{FLT_MAX, FLT_MAX, FLT_MAX}, {-FLT_MAX, -FLT_MAX, -FLT_MAX}};
 }
-__device__ __forceinline__ float unordered(uint32_t u) {
-    return __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
+__device__ __forceinline__ Box6 unite(const Box6& a, const Box6& b) {
+    Box6 u;
+    for (int c = 0; c < 3; ++c) {
+        u.lo[c] = fminf(a.lo[c], b.lo[c]);
+        u.hi[c] = fmaxf(a.hi[c], b.hi[c]);
+    }
+    return u;
+}
+// The union of the workgroup's boxes, in thread 0.
+__device__ __forceinline__ Box6 block_unite(Box6 b) {
+    __shared__ Box6 waves[kBlock / 64];
+    for (int off = 32; off > 0; off >>= 1) {
+        Box6 o;
+        for (int c = 0; c < 3; ++c) {
+            o.lo[c] = __shfl_xor(b.lo[c], off);
+            o.hi[c] = __shfl_xor(b.hi[c], off);
+        }
+        b = unite(b, o);
+    }
+    if (__lane_id() == 0) waves[threadIdx.x / 64] = b;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < kBlock / 64; ++w) b = unite(b, waves[w]);
+    return b;
 }
 
-// 1. triangle boxes and the bounds of their centroids
+// 1. triangle boxes, and per workgroup the bounds of their centroids. One
+// set of bounds per workgroup of at most kBoundBlocks, reduced by one more
+// workgroup: with six same-address atomics per 256 triangles this pass took
+// 355 us at 1.31M triangles, against 19 us (and 4 us for the reduction).
+constexpr int kBoundBlocks = 1024;
 __global__ void __launch_bounds__(kBlock) k_tri_boxes(const float* __restrict__ pos, const int32_t* __restrict__ idx,
-                                                      int64_t nt, Box6* __restrict__ boxes,
-                                                      uint32_t* __restrict__ cbounds) {
-    __shared__ float red[6][kBlock];
-    int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    float c[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, C[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-    if (i < nt) {
-        Box6 b;
-        for (int k = 0; k < 3; ++k) { b.lo[k] = FLT_MAX; b.hi[k] = -FLT_MAX; }
+                                                      int64_t nt, Box6* __restrict__ boxes, Box6* __restrict__ partial) {
+    Box6 all = empty_box();
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < nt; i += (int64_t)gridDim.x * kBlock) {
+        Box6 b = empty_box();
         for (int v = 0; v < 3; ++v) {
             const float* p = pos + 3 * (int64_t)idx[3 * i + v];
             for (int k = 0; k < 3; ++k) { b.lo[k] = fminf(b.lo[k], p[k]); b.hi[k] = fmaxf(b.hi[k], p[k]); }
         }
         boxes[i] = b;
-        for (int k = 0; k < 3; ++k) c[k] = C[k] = 0.5f * (b.lo[k] + b.hi[k]);
+        Box6 c;
+        for (int k = 0; k < 3; ++k) c.lo[k] = c.hi[k] = 0.5f * (b.lo[k] + b.hi[k]);
+        all = unite(all, c);
     }
-    for (int k = 0; k < 3; ++k) { red[k][threadIdx.x] = c[k]; red[3 + k][threadIdx.x] = C[k]; }
-    __syncthreads();
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            for (int k = 0; k < 3; ++k) {
-                red[k][threadIdx.x] = fminf(red[k][threadIdx.x], red[k][threadIdx.x + s]);
-                red[3 + k][threadIdx.x] = fmaxf(red[3 + k][threadIdx.x], red[3 + k][threadIdx.x + s]);
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        for (int k = 0; k < 3; ++k) {
-            atomicMin(&cbounds[k], ordered(red[k][0]));
-            atomicMax(&cbounds[3 + k], ordered(red[3 + k][0]));
-        }
-    }
+    all = block_unite(all);
+    if (threadIdx.x == 0) partial[blockIdx.x] = all;
+}
+// One workgroup: the union of n boxes.
+__global__ void __launch_bounds__(kBlock) k_unite(const Box6* __restrict__ boxes, int n, Box6* __restrict__ out) {
+    Box6 all = empty_box();
+    for (int i = threadIdx.x; i < n; i += kBlock) all = unite(all, boxes[i]);
+    all = block_unite(all);
+    if (threadIdx.x == 0) *out = all;
 }
 
 __device__ __forceinline__ uint64_t spread21(uint64_t x) {
@@ -92,14 +106,14 @@ __device__ __forceinline__ uint64_t spread21(uint64_t x) {
 
 // 2. Morton codes of centroids in the centroid bounds
 __global__ void __launch_bounds__(kBlock) k_morton(const Box6* __restrict__ boxes, int64_t nt,
-                                                   const uint32_t* __restrict__ cbounds, uint64_t* __restrict__ codes,
+                                                   const Box6* __restrict__ cbounds, uint64_t* __restrict__ codes,
                                                    int32_t* __restrict__ ids) {
     int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= nt) return;
     const Box6 b = boxes[i];
     uint64_t q[3];
     for (int k = 0; k < 3; ++k) {
-        float lo = unordered(cbounds[k]), hi = unordered(cbounds[3 + k]);
+        float lo = cbounds->lo[k], hi = cbounds->hi[k];
         float c = 0.5f * (b.lo[k] + b.hi[k]);
         float e = hi - lo;
         float u = e > 0.0f ? (c - lo) / e : 0.5f;
@@ -119,11 +133,56 @@ __device__ __forceinline__ int delta(const uint64_t* __restrict__ k, int32_t n, 
     return 64 + __clz((int)((uint32_t)i ^ (uint32_t)j));
 }
 
-// 3. internal node i of n-1; nodes 0..n-2 internal, n-1.. leaves (leaf k = n-1+k)
-__global__ void __launch_bounds__(kBlock) k_karras(const uint64_t* __restrict__ keys, int32_t n,
+// 3. The union of every aligned run of 2^j of the n boxes `in`, j = 1 ..
+// levels, written at out[j - 1]. The first pass gathers the leaf boxes (ids
+// given) and stores them in sorted order. A workgroup covers 256 boxes and
+// their eight levels in LDS.
+constexpr int kRunLevels = 8;
+struct RunArgs {
+    const Box6* in;
+    const int32_t* ids;  // first pass: in[ids[k]] is box k; null: in[k]
+    Box6* sorted;        // first pass: box k to sorted[k]
+    int32_t n, levels;
+    Box6* out[kRunLevels];
+};
+__global__ void __launch_bounds__(kBlock) k_runs(RunArgs a) {
+    __shared__ Box6 run[kBlock];
+    const int32_t t = threadIdx.x, k = blockIdx.x * kBlock + t;
+    Box6 b = empty_box();
+    if (k < a.n) {
+        b = a.in[a.ids ? a.ids[k] : k];
+        if (a.ids) a.sorted[k] = b;
+    }
+    run[t] = b;
+    int32_t count = a.n;
+    for (int j = 0; j < a.levels; ++j) {
+        const int32_t width = kBlock >> (j + 1), at = blockIdx.x * width + t;
+        count = (count + 1) / 2;
+        __syncthreads();
+        if (t < width) b = unite(run[2 * t], run[2 * t + 1]);
+        __syncthreads();
+        if (t < width) {
+            run[t] = b;
+            if (at < count) a.out[j][at] = b;
+        }
+    }
+}
+
+// 4. Internal node i of n-1, its children, range of leaves and box; nodes
+// 0..n-2 internal, n-1.. leaves (leaf k = n-1+k). A range is made of at most
+// two runs per level (mostly few: half of the nodes hold two or three
+// leaves). Climbing from the leaves instead, the second child to arrive
+// uniting the boxes, needs an acquire and a release at device scope at every
+// step, which write back and invalidate the caches of the eight XCDs: 5.1 ms
+// at 1.31M triangles, against 30 us for the runs and 27 us more here.
+constexpr int kMaxRunLevels = 27;  // fewer than 2^26 leaves
+struct Runs {
+    const Box6* level[kMaxRunLevels];  // [0] the sorted leaf boxes
+};
+__global__ void __launch_bounds__(kBlock) k_karras(const uint64_t* __restrict__ keys, int32_t n, Runs runs,
                                                    int32_t* __restrict__ left, int32_t* __restrict__ right,
-                                                   int32_t* __restrict__ parent, int32_t* __restrict__ range_lo,
-                                                   int32_t* __restrict__ range_hi) {
+                                                   int32_t* __restrict__ range_lo, int32_t* __restrict__ range_hi,
+                                                   Box6* __restrict__ boxes) {
     int32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n - 1) return;
     int d = (delta(keys, n, i, i + 1) - delta(keys, n, i, i - 1)) >= 0 ? 1 : -1;
@@ -144,35 +203,17 @@ __global__ void __launch_bounds__(kBlock) k_karras(const uint64_t* __restrict__ 
     } while (t > 1);
     int32_t gamma = i + s * d + min(d, 0);
     int32_t lo = min(i, j), hi = max(i, j);
-    int32_t lc = (lo == gamma) ? (n - 1 + gamma) : gamma;
-    int32_t rc = (hi == gamma + 1) ? (n - 1 + gamma + 1) : (gamma + 1);
-    left[i] = lc;
-    right[i] = rc;
-    parent[lc] = i;
-    parent[rc] = i;
+    left[i] = (lo == gamma) ? (n - 1 + gamma) : gamma;
+    right[i] = (hi == gamma + 1) ? (n - 1 + gamma + 1) : (gamma + 1);
     range_lo[i] = lo;
     range_hi[i] = hi;
-}
-
-// 4. bottom-up boxes; flags start at zero
-__global__ void __launch_bounds__(kBlock) k_refit(const Box6* __restrict__ tri_boxes, const int32_t* __restrict__ ids,
-                                                  int32_t n, const int32_t* __restrict__ left,
-                                                  const int32_t* __restrict__ right, const int32_t* __restrict__ parent,
-                                                  Box6* nodes, uint32_t* flags) {
-    int32_t k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= n) return;
-    int32_t node = n - 1 + k;
-    nodes[node] = tri_boxes[ids[k]];
-    int32_t p = parent[node];
-    while (p >= 0) {
-        // release this subtree's box; the second arrival acquires its sibling's
-        uint32_t prev = __hip_atomic_fetch_add(&flags[p], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (prev == 0) return;
-        Box6 a = nodes[left[p]], b = nodes[right[p]], u;
-        for (int c = 0; c < 3; ++c) { u.lo[c] = fminf(a.lo[c], b.lo[c]); u.hi[c] = fmaxf(a.hi[c], b.hi[c]); }
-        nodes[p] = u;
-        p = parent[p];
+    Box6 box = empty_box();
+    int32_t a = lo, b = hi + 1;
+    for (int lv = 0; a < b; ++lv, a >>= 1, b >>= 1) {
+        if (a & 1) box = unite(box, runs.level[lv][a++]);
+        if (b & 1) box = unite(box, runs.level[lv][--b]);
     }
+    boxes[i] = box;
 }
 
 __device__ __forceinline__ float area6(const Box6& b) {
@@ -180,19 +221,22 @@ __device__ __forceinline__ float area6(const Box6& b) {
     return 2.0f * (dx * dy + dy * dz + dz * dx);
 }
 
+// Counters of the collapse, read back by the host after every few levels.
+constexpr int kMaxLevels = 128;  // a Karras tree over 63 + 32 key bits is shallower
+struct CollapseCounts {
+    uint32_t items[kMaxLevels + 1];  // wide nodes of each level
+    uint32_t max_leaf;
+    double cost;
+};
+
 struct CollapseArgs {
-    int32_t n, max_leaf;
+    int32_t n, max_leaf, level;
     const int32_t *left, *right, *range_lo, *range_hi;
     const Box6* nodes;
     WideNode<4>* wide;
-    const int2* qin;           // (bvh2 node, wide node)
-    const uint32_t* qin_count;
-    int2* qout;
-    uint32_t* qout_count;
-    uint32_t* wide_count;
-    uint32_t* max_leaf_seen;
-    double* cost;
-    float inv_root_area;
+    const int32_t* qin;   // binary nodes of this level's wide nodes, in order
+    int32_t* qout;        // and of the next level's
+    CollapseCounts* counts;
 };
 
 __device__ __forceinline__ int32_t subtree_size(const CollapseArgs& a, int32_t node) {
@@ -202,54 +246,127 @@ __device__ __forceinline__ bool leafable(const CollapseArgs& a, int32_t node) {
     return node >= a.n - 1 || subtree_size(a, node) <= a.max_leaf;
 }
 
-// 5. one level of the collapse: one thread per wide node of this level
+// 5. one level of the collapse: one thread per wide node of this level. A
+// level's wide nodes are numbered in queue order after those of the levels
+// above, so a child's number follows from its place in the next queue, and a
+// workgroup takes its places with one atomic (and adds to the cost and the
+// largest leaf with one each at its end): one same-address atomic per child,
+// node and leaf made the levels of 1.31M triangles 650 us, against 200 us.
+// The grid does not depend on the level's size, which the host does not wait
+// for: workgroups without work leave at once.
 __global__ void __launch_bounds__(kBlock) k_collapse(CollapseArgs a) {
-    uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-    if (t >= *a.qin_count) return;
-    const int2 item = a.qin[t];
-    int32_t kids[4] = {a.left[item.x], a.right[item.x], -1, -1};
-    int nk = 2;
-    while (nk < 4) {
-        int best = -1;
-        float best_a = -1.0f;
-        for (int k = 0; k < nk; ++k) {
-            if (leafable(a, kids[k])) continue;
-            float ar = area6(a.nodes[kids[k]]);
-            if (ar > best_a) { best_a = ar; best = k; }
+    __shared__ uint32_t s_sum[2][kBlock / 64], s_base[2];
+    __shared__ double s_cost[kBlock / 64];
+    __shared__ uint32_t s_leaf[kBlock / 64];
+    const uint32_t items = a.counts->items[a.level];
+    if (blockIdx.x * kBlock >= items) return;
+    uint32_t first = 0;  // number of this level's first wide node
+    for (int l = 0; l < a.level; ++l) first += a.counts->items[l];
+    const Box6 root = a.nodes[0];
+    const float ra = area6(root), inv_root_area = ra > 0 ? 1.0f / ra : 0.0f;
+    const int lane = (int)__lane_id(), wave = threadIdx.x / 64;
+    double cost = 0;
+    uint32_t max_leaf = 0;
+    int par = 0;
+    for (uint32_t base = blockIdx.x * kBlock; base < items; base += gridDim.x * kBlock, par ^= 1) {
+        const uint32_t t = base + threadIdx.x;
+        const bool live = t < items;
+        int32_t kids[4] = {-1, -1, -1, -1};
+        int nk = 0;
+        uint32_t inner = 0;  // bit k: child k is a wide node of the next level
+        if (live) {
+            const int32_t node = a.qin[t];
+            kids[0] = a.left[node];
+            kids[1] = a.right[node];
+            nk = 2;
+            while (nk < 4) {
+                int best = -1;
+                float best_a = -1.0f;
+                for (int k = 0; k < nk; ++k) {
+                    if (leafable(a, kids[k])) continue;
+                    float ar = area6(a.nodes[kids[k]]);
+                    if (ar > best_a) { best_a = ar; best = k; }
+                }
+                if (best < 0) break;
+                int32_t open = kids[best];
+                kids[best] = a.left[open];
+                kids[nk++] = a.right[open];
+            }
+            for (int k = 0; k < nk; ++k) inner |= leafable(a, kids[k]) ? 0u : 1u << k;
+            cost += (double)area6(a.nodes[node]) * inv_root_area;
         }
-        if (best < 0) break;
-        int32_t open = kids[best];
-        kids[best] = a.left[open];
-        kids[nk++] = a.right[open];
+        // places in the next queue: within the wave, the workgroup, the level
+        const uint32_t mine = (uint32_t)__popc(inner);
+        uint32_t incl = mine;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t v = __shfl_up(incl, off);
+            if (lane >= off) incl += v;
+        }
+        if (lane == 63) s_sum[par][wave] = incl;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint32_t total = 0;
+            for (int w = 0; w < kBlock / 64; ++w) total += s_sum[par][w];
+            s_base[par] = total ? atomicAdd(&a.counts->items[a.level + 1], total) : 0u;
+        }
+        __syncthreads();
+        uint32_t place = s_base[par] + incl - mine;
+        for (int w = 0; w < wave; ++w) place += s_sum[par][w];
+        if (!live) continue;
+        WideNode<4> w;
+        for (int k = 0; k < 4; ++k) {
+            if (k >= nk) {
+                w.lox[k] = w.loy[k] = w.loz[k] = w.hix[k] = w.hiy[k] = w.hiz[k] = FLT_MAX;
+                w.child[k] = make_leaf(0, 0);
+                continue;
+            }
+            const int32_t c = kids[k];
+            const Box6 b = a.nodes[c];
+            w.lox[k] = b.lo[0]; w.hix[k] = b.hi[0];
+            w.loy[k] = b.lo[1]; w.hiy[k] = b.hi[1];
+            w.loz[k] = b.lo[2]; w.hiz[k] = b.hi[2];
+            if (inner >> k & 1u) {
+                a.qout[place] = c;
+                w.child[k] = first + items + place;
+                ++place;
+            } else {
+                const int32_t at = c >= a.n - 1 ? c - (a.n - 1) : a.range_lo[c];
+                const int32_t cnt = subtree_size(a, c);
+                w.child[k] = make_leaf((uint32_t)at, (uint32_t)cnt);
+                max_leaf = max(max_leaf, (uint32_t)cnt);
+                cost += (double)area6(b) * inv_root_area * cnt;
+            }
+        }
+        a.wide[first + t] = w;
     }
-    WideNode<4> w;
-    double cost = (double)area6(a.nodes[item.x]) * a.inv_root_area;
-    for (int k = 0; k < 4; ++k) {
-        if (k >= nk) {
-            w.lox[k] = w.loy[k] = w.loz[k] = w.hix[k] = w.hiy[k] = w.hiz[k] = FLT_MAX;
-            w.child[k] = make_leaf(0, 0);
-            continue;
-        }
-        const int32_t c = kids[k];
-        const Box6 b = a.nodes[c];
-        w.lox[k] = b.lo[0]; w.hix[k] = b.hi[0];
-        w.loy[k] = b.lo[1]; w.hiy[k] = b.hi[1];
-        w.loz[k] = b.lo[2]; w.hiz[k] = b.hi[2];
-        if (leafable(a, c)) {
-            int32_t first = c >= a.n - 1 ? c - (a.n - 1) : a.range_lo[c];
-            int32_t cnt = subtree_size(a, c);
-            w.child[k] = make_leaf((uint32_t)first, (uint32_t)cnt);
-            atomicMax(a.max_leaf_seen, (uint32_t)cnt);
-            cost += (double)area6(b) * a.inv_root_area * cnt;
-        } else {
-            uint32_t slot = atomicAdd(a.wide_count, 1u);
-            uint32_t q = atomicAdd(a.qout_count, 1u);
-            a.qout[q] = make_int2(c, (int)slot);
-            w.child[k] = slot;
-        }
+    for (int off = 32; off > 0; off >>= 1) {
+        cost += __shfl_xor(cost, off);
+        max_leaf = max(max_leaf, (uint32_t)__shfl_xor((int)max_leaf, off));
     }
-    a.wide[item.y] = w;
-    atomicAdd(a.cost, cost);
+    if (lane == 0) {
+        s_cost[wave] = cost;
+        s_leaf[wave] = max_leaf;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / 64; ++w) {
+            cost += s_cost[w];
+            max_leaf = max(max_leaf, s_leaf[w]);
+        }
+        atomicAdd(&a.counts->cost, cost);
+        atomicMax(&a.counts->max_leaf, max_leaf);
+    }
+}
+
+// Before the first level: one item, the root, nothing counted.
+__global__ void k_collapse_begin(CollapseCounts* c, int32_t* q) {
+    const int t = threadIdx.x;
+    if (t <= kMaxLevels) c->items[t] = t == 0 ? 1u : 0u;
+    if (t == 0) {
+        c->max_leaf = 0u;
+        c->cost = 0.0;
+        q[0] = 0;
+    }
 }
 
 // 6. triangles in Morton order: (v0, original index), (v1, 0), (v2, 0)
@@ -272,11 +389,6 @@ __global__ void __launch_bounds__(kBlock) k_quantize(const WideNode<4>* __restri
     QNode4 q;
     quantize_node(in[i], q);
     out[i] = q;
-}
-
-__global__ void k_init_u32(uint32_t* p, int64_t n, uint32_t v) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
 }
 
 inline unsigned blocks_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -306,18 +418,16 @@ int build_lbvh(ilm_mesh* m, int max_leaf, int node_format) {
     };
     float *d_pos = nullptr;
     int32_t *d_idx = nullptr, *ids_in = nullptr, *ids = nullptr, *left = nullptr, *right = nullptr,
-            *parent = nullptr, *rlo = nullptr, *rhi = nullptr;
+            *rlo = nullptr, *rhi = nullptr, *qa = nullptr, *qb = nullptr;
     uint64_t *codes_in = nullptr, *codes = nullptr;
-    Box6 *tri_boxes = nullptr, *nodes = nullptr;
-    uint32_t *cb = nullptr, *flags = nullptr, *counts = nullptr;
-    int2 *qa = nullptr, *qb = nullptr;
-    double* cost = nullptr;
+    Box6 *tri_boxes = nullptr, *nodes = nullptr, *runs = nullptr, *cb = nullptr;
+    CollapseCounts* counts = nullptr;
     const int32_t ninner = std::max(n - 1, 1);
     int rc = ILM_OK;
     rc |= alloc(nv * 3 * sizeof(float), (void**)&d_pos);
     rc |= alloc(nt * 3 * sizeof(int32_t), (void**)&d_idx);
     rc |= alloc(nt * sizeof(Box6), (void**)&tri_boxes);
-    rc |= alloc(6 * sizeof(uint32_t), (void**)&cb);
+    rc |= alloc((kBoundBlocks + 1) * sizeof(Box6), (void**)&cb);  // centroid bounds, then the workgroups'
     rc |= alloc(nt * sizeof(uint64_t), (void**)&codes_in);
     rc |= alloc(nt * sizeof(uint64_t), (void**)&codes);
     rc |= alloc(nt * sizeof(int32_t), (void**)&ids_in);
@@ -326,13 +436,11 @@ int build_lbvh(ilm_mesh* m, int max_leaf, int node_format) {
     rc |= alloc(ninner * sizeof(int32_t), (void**)&right);
     rc |= alloc(ninner * sizeof(int32_t), (void**)&rlo);
     rc |= alloc(ninner * sizeof(int32_t), (void**)&rhi);
-    rc |= alloc((2 * nt) * sizeof(int32_t), (void**)&parent);
     rc |= alloc((2 * nt) * sizeof(Box6), (void**)&nodes);
-    rc |= alloc(ninner * sizeof(uint32_t), (void**)&flags);
-    rc |= alloc(ninner * sizeof(int2), (void**)&qa);
-    rc |= alloc(ninner * sizeof(int2), (void**)&qb);
-    rc |= alloc(8 * sizeof(uint32_t), (void**)&counts);  // [0] qa, [1] qb, [2] wide, [3] max leaf
-    rc |= alloc(sizeof(double), (void**)&cost);
+    rc |= alloc((nt + kMaxRunLevels) * sizeof(Box6), (void**)&runs);
+    rc |= alloc(ninner * sizeof(int32_t), (void**)&qa);
+    rc |= alloc(ninner * sizeof(int32_t), (void**)&qb);
+    rc |= alloc(sizeof(CollapseCounts), (void**)&counts);
     if (rc != ILM_OK) { cleanup(); return fail(ILM_ERR_NOMEM, "LBVH scratch allocation failed"); }
     // wide nodes: at most one per internal BVH2 node, plus the root
     void* d_nodes = nullptr;
@@ -366,14 +474,10 @@ int build_lbvh(ilm_mesh* m, int max_leaf, int node_format) {
     LBVH_HIP(hipMemcpyAsync(d_pos, m->pos.data(), nv * 3 * sizeof(float), hipMemcpyHostToDevice, st));
     LBVH_HIP(hipMemcpyAsync(d_idx, m->idx.data(), nt * 3 * sizeof(int32_t), hipMemcpyHostToDevice, st));
     LBVH_HIP(hipEventRecord(e0, st));
-    const uint32_t cb_init[6] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0u, 0u, 0u};
-    // small initialisations by kernel (no memset nodes if a caller captures the stream)
-    hipLaunchKernelGGL(k_init_u32, dim3(1), dim3(64), 0, st, cb, 3, cb_init[0]);
-    hipLaunchKernelGGL(k_init_u32, dim3(1), dim3(64), 0, st, cb + 3, 3, 0u);
-    hipLaunchKernelGGL(k_init_u32, dim3(blocks_for(ninner)), dim3(kBlock), 0, st, flags, (int64_t)ninner, 0u);
-    hipLaunchKernelGGL(k_init_u32, dim3(1), dim3(64), 0, st, counts, 8, 0u);
-    hipLaunchKernelGGL(k_init_u32, dim3(1), dim3(64), 0, st, (uint32_t*)cost, 2, 0u);
-    hipLaunchKernelGGL(k_tri_boxes, dim3(blocks_for(nt)), dim3(kBlock), 0, st, d_pos, d_idx, nt, tri_boxes, cb);
+    const int bound_blocks = (int)std::min<int64_t>(blocks_for(nt), kBoundBlocks);
+    hipLaunchKernelGGL(k_tri_boxes, dim3((unsigned)bound_blocks), dim3(kBlock), 0, st, d_pos, d_idx, nt, tri_boxes,
+                       cb + 1);
+    hipLaunchKernelGGL(k_unite, dim3(1), dim3(kBlock), 0, st, cb + 1, bound_blocks, cb);
     hipLaunchKernelGGL(k_morton, dim3(blocks_for(nt)), dim3(kBlock), 0, st, tri_boxes, nt, cb, codes_in, ids_in);
     LBVH_HIP(hipGetLastError());
     size_t sort_bytes = 0;
@@ -383,8 +487,10 @@ int build_lbvh(ilm_mesh* m, int max_leaf, int node_format) {
     LBVH_HIP(hipcub::DeviceRadixSort::SortPairs(sort_tmp, sort_bytes, codes_in, codes, ids_in, ids, n, 0, 63, st));
 
     int levels = 0;
-    uint32_t h_counts[8] = {0};
-    double h_cost = 0;
+    int64_t nwide = 0;
+    CollapseCounts h;
+    h.max_leaf = 0;
+    h.cost = 0;
     if (n <= max_leaf) {
         // a single leaf under the root
         WideNode<4> w;
@@ -404,60 +510,66 @@ int build_lbvh(ilm_mesh* m, int max_leaf, int node_format) {
         w.hix[0] = hi[0]; w.hiy[0] = hi[1]; w.hiz[0] = hi[2];
         w.child[0] = make_leaf(0, (uint32_t)n);
         LBVH_HIP(hipMemcpyAsync(d_nodes, &w, sizeof w, hipMemcpyHostToDevice, st));
-        h_counts[2] = 1;
-        h_counts[3] = (uint32_t)n;
-        h_cost = (double)n;
+        nwide = 1;
+        h.max_leaf = (uint32_t)n;
+        h.cost = (double)n;
         levels = 1;
     } else {
-        hipLaunchKernelGGL(k_init_u32, dim3(blocks_for(2 * nt)), dim3(kBlock), 0, st, (uint32_t*)parent, 2 * nt,
-                           0xFFFFFFFFu);
-        hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1)), dim3(kBlock), 0, st, codes, n, left, right, parent,
-                           rlo, rhi);
-        hipLaunchKernelGGL(k_refit, dim3(blocks_for(n)), dim3(kBlock), 0, st, tri_boxes, ids, n, left, right, parent,
-                           nodes, flags);
+        // runs of 2, 4, ... leaves, eight levels per pass until one box is left
+        Runs tree{};
+        tree.level[0] = nodes + (n - 1);
+        Box6* at = runs;
+        int32_t count = n;
+        for (int lv = 0; count > 1;) {
+            RunArgs r{};
+            r.in = lv == 0 ? tri_boxes : tree.level[lv];
+            r.ids = lv == 0 ? ids : nullptr;
+            r.sorted = nodes + (n - 1);
+            r.n = count;
+            const unsigned blocks = blocks_for(count);
+            while (r.levels < kRunLevels && count > 1) {
+                count = (count + 1) / 2;
+                tree.level[++lv] = r.out[r.levels++] = at;
+                at += count;
+            }
+            hipLaunchKernelGGL(k_runs, dim3(blocks), dim3(kBlock), 0, st, r);
+        }
+        hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1)), dim3(kBlock), 0, st, codes, n, tree, left, right, rlo,
+                           rhi, nodes);
+        hipLaunchKernelGGL(k_collapse_begin, dim3(1), dim3(kBlock), 0, st, counts, qa);
         LBVH_HIP(hipGetLastError());
-        Box6 root;
-        LBVH_HIP(hipMemcpyAsync(&root, nodes, sizeof root, hipMemcpyDeviceToHost, st));
-        LBVH_HIP(hipStreamSynchronize(st));
-        float ra = 2.0f * ((root.hi[0] - root.lo[0]) * (root.hi[1] - root.lo[1]) +
-                           (root.hi[1] - root.lo[1]) * (root.hi[2] - root.lo[2]) +
-                           (root.hi[2] - root.lo[2]) * (root.hi[0] - root.lo[0]));
-        // level 0: internal node 0 -> wide node 0
-        const int2 first = make_int2(0, 0);
-        const uint32_t one[3] = {1u, 0u, 1u};  // qa count, qb count, wide count
-        LBVH_HIP(hipMemcpyAsync(qa, &first, sizeof first, hipMemcpyHostToDevice, st));
-        LBVH_HIP(hipMemcpyAsync(counts, one, sizeof one, hipMemcpyHostToDevice, st));
         CollapseArgs a;
         a.n = n;
         a.max_leaf = max_leaf;
         a.left = left; a.right = right; a.range_lo = rlo; a.range_hi = rhi;
         a.nodes = nodes;
         a.wide = reinterpret_cast<WideNode<4>*>(d_nodes);
-        a.wide_count = counts + 2;
-        a.max_leaf_seen = counts + 3;
-        a.cost = cost;
-        a.inv_root_area = ra > 0 ? 1.0f / ra : 0.0f;
-        uint32_t level_items = 1;
-        int2 *qin = qa, *qout = qb;
-        uint32_t *cin = counts, *cout = counts + 1;
-        while (level_items > 0) {
-            if (++levels > 4096) return fail_all(ILM_ERR_STATE, "LBVH collapse did not terminate");
-            a.qin = qin; a.qin_count = cin; a.qout = qout; a.qout_count = cout;
-            hipLaunchKernelGGL(k_init_u32, dim3(1), dim3(64), 0, st, cout, 1, 0u);
-            hipLaunchKernelGGL(k_collapse, dim3(blocks_for(level_items)), dim3(kBlock), 0, st, a);
+        a.counts = counts;
+        int32_t *qin = qa, *qout = qb;
+        const unsigned grid = (unsigned)std::min<int64_t>(blocks_for(n), (int64_t)ctx->cu_count * 8);
+        // a balanced tree's levels and a few more before the first wait
+        int until = 4;
+        for (int64_t m = n; m > max_leaf; m /= 4) ++until;
+        for (;;) {
+            for (; levels < until; ++levels) {
+                a.level = levels;
+                a.qin = qin; a.qout = qout;
+                hipLaunchKernelGGL(k_collapse, dim3(grid), dim3(kBlock), 0, st, a);
+                std::swap(qin, qout);
+            }
             LBVH_HIP(hipGetLastError());
-            LBVH_HIP(hipMemcpyAsync(&level_items, cout, sizeof level_items, hipMemcpyDeviceToHost, st));
+            LBVH_HIP(hipMemcpyAsync(&h, counts, sizeof h, hipMemcpyDeviceToHost, st));
             LBVH_HIP(hipStreamSynchronize(st));
-            std::swap(qin, qout);
-            std::swap(cin, cout);
+            if (h.items[levels] == 0) break;
+            if (levels == kMaxLevels) return fail_all(ILM_ERR_STATE, "LBVH collapse did not terminate");
+            until = std::min(levels + 4, kMaxLevels);
         }
-        LBVH_HIP(hipMemcpyAsync(h_counts, counts, sizeof h_counts, hipMemcpyDeviceToHost, st));
-        LBVH_HIP(hipMemcpyAsync(&h_cost, cost, sizeof h_cost, hipMemcpyDeviceToHost, st));
+        while (levels > 0 && h.items[levels - 1] == 0) --levels;
+        for (int l = 0; l < levels; ++l) nwide += h.items[l];
     }
     hipLaunchKernelGGL(k_pack, dim3(blocks_for(n)), dim3(kBlock), 0, st, d_pos, d_idx, ids, n,
                        reinterpret_cast<float4*>(d_tris));
     LBVH_HIP(hipGetLastError());
-    const int64_t nwide = h_counts[2];
     size_t stride = sizeof(WideNode<4>);
     if (node_format == ILM_NODES_QUANTIZED) {
         void* qn = nullptr;
@@ -500,10 +612,10 @@ int build_lbvh(ilm_mesh* m, int max_leaf, int node_format) {
     m->info.tri_bytes = nt * 12 * (int64_t)sizeof(float);
     m->info.width = 4;
     m->info.depth = levels;
-    m->info.max_leaf = (int32_t)h_counts[3];
+    m->info.max_leaf = (int32_t)h.max_leaf;
     m->info.stack_need = 3 * levels + 1;  // at most three deferred siblings per level
     m->info.build_ms = gpu_ms;
-    m->info.sah_cost = h_cost;
+    m->info.sah_cost = h.cost;
     m->built = true;
     return ILM_OK;
 }

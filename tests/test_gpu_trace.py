@@ -345,6 +345,46 @@ def _classify_disagreements(orc, om, pos, idx, rays, ph, th, pc, tc):
     return ns.mean(), (ns.sum() + out["bvhmesh"]) / n, out, others, zero_dir
 
 
+@pytest.mark.parametrize("ntri", [5, 8, 255, 256, 257, 511, 513, 65535, 65537, 140001])
+def test_lbvh_boxes_are_tight(ntri, gpu_ctx, ilm):
+    """Every child's box is exactly the union of its triangles' boxes (unions
+    of floats do not round), at triangle counts around the aligned runs of 256
+    and 65,536 sorted leaves that the boxes are made from; the reported
+    largest leaf and depth are those of the tree."""
+    pos, idx = meshgen.random_triangles(ntri, seed=ntri, extent=2.0, size=0.05)
+    m = ilm.Mesh(gpu_ctx, pos, idx)
+    info = m.build(builder=ilm.ILM_BUILDER_LBVH, max_leaf=3)
+    nodes, order = m.export()
+    boxes, child = ilm.decode_bvh4(nodes)
+    tri = pos[idx]
+    tlo, thi = tri.min(axis=1), tri.max(axis=1)
+    levels, largest, seen = [np.array([0])], 0, 0
+    while len(levels[-1]):
+        c = child[levels[-1]]
+        levels.append(c[(c & 0x80000000) == 0])
+    lo, hi = np.full((len(boxes), 3), np.inf, np.float32), np.full((len(boxes), 3), -np.inf, np.float32)
+    for level in reversed(levels[:-1]):
+        for k in range(4):
+            c = child[level, k]
+            blo, bhi = np.full((len(level), 3), np.inf, np.float32), np.full((len(level), 3), -np.inf, np.float32)
+            leaf = (c & 0x80000000) != 0
+            blo[~leaf], bhi[~leaf] = lo[c[~leaf]], hi[c[~leaf]]
+            cnt, first = c & 31, (c & 0x7FFFFFFF) >> 5
+            for j in range(int(cnt[leaf].max(initial=0))):
+                has = leaf & (cnt > j)
+                ids = order[first[has] + j]
+                blo[has], bhi[has] = np.minimum(blo[has], tlo[ids]), np.maximum(bhi[has], thi[ids])
+                seen += int(has.sum())
+            largest = max(largest, int(cnt[leaf].max(initial=0)))
+            used = ~leaf | (cnt > 0)
+            assert np.array_equal(blo[used], boxes[level, k, :3][used])
+            assert np.array_equal(bhi[used], boxes[level, k, 3:][used])
+            lo[level], hi[level] = np.minimum(lo[level], blo), np.maximum(hi[level], bhi)
+    assert seen == ntri and sum(len(x) for x in levels) == info["nodes"]
+    assert info["depth"] == len(levels) - 1 and info["max_leaf"] == largest
+    m.close()
+
+
 @pytest.mark.parametrize("kind", ["primary", "incoherent"])
 def test_c2_closest_matches_oracle_bvhmesh(c2, c2_oracle, gpu_ctx, ilm, orc, kind):
     """1,334,720 triangles: GPU closest hit vs the oracle's BVHMesh (reference
