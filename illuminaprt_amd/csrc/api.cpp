@@ -42,6 +42,26 @@ int ensure_spill(ilm_ctx* ctx, size_t words) {
     return ILM_OK;
 }
 
+int ensure_build_ws(ilm_ctx* ctx, size_t bytes) {
+    if (ctx->build_bytes >= bytes) return ILM_OK;
+    ILM_HIP(hipSetDevice(ctx->device));
+    if (ctx->build_ws) {
+        ILM_HIP(hipStreamSynchronize(ctx->stream));
+        ILM_HIP(hipFree(ctx->build_ws));
+        ctx->build_ws = nullptr;
+        ctx->build_bytes = 0;
+    }
+    hipError_t e = hipMalloc(&ctx->build_ws, bytes);
+    if (e != hipSuccess) {
+        ctx->build_ws = nullptr;
+        return e == hipErrorOutOfMemory
+                   ? fail(ILM_ERR_NOMEM, "device allocation of " + std::to_string(bytes) + " bytes")
+                   : fail_hip(e, "hipMalloc");
+    }
+    ctx->build_bytes = bytes;
+    return ILM_OK;
+}
+
 }  // namespace ilm
 
 using ilm::fail;
@@ -94,6 +114,7 @@ int ilm_ctx_destroy(ilm_ctx* ctx) {
     for (void* p : ctx->allocs) (void)hipFree(p);
     for (hipEvent_t ev : ctx->events) (void)hipEventDestroy(ev);
     if (ctx->spill) (void)hipFree(ctx->spill);
+    if (ctx->build_ws) (void)hipFree(ctx->build_ws);
     if (ctx->counters) (void)hipFree(ctx->counters);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -127,6 +148,18 @@ int ilm_alloc(ilm_ctx* ctx, size_t bytes, void** dev) {
     ILM_HIP(hipSetDevice(ctx->device));
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        // the kept build workspace makes room, unless a build uses it
+        ilm::BuildWorkspace held(ctx, true);
+        if (held.mine && ctx->build_ws) {
+            (void)hipGetLastError();
+            ILM_HIP(hipStreamSynchronize(ctx->stream));
+            ILM_HIP(hipFree(ctx->build_ws));
+            ctx->build_ws = nullptr;
+            ctx->build_bytes = 0;
+            e = hipMalloc(&p, bytes);
+        }
+    }
     if (e == hipErrorOutOfMemory) return fail(ILM_ERR_NOMEM, "device allocation of " + std::to_string(bytes) + " bytes");
     if (e != hipSuccess) return ilm::fail_hip(e, "hipMalloc");
     std::lock_guard<std::mutex> g(ctx->mu);

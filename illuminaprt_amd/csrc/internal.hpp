@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <chrono>
 #include <mutex>
 #include <set>
@@ -51,6 +52,13 @@ struct ilm_ctx {
     uint32_t* spill = nullptr;
     size_t spill_words = 0;
     uint64_t spill_generation = 0;  // counts reallocations of spill (graphs key on it)
+    // scratch of the device builder, grown on demand up to kBuildKeep bytes and
+    // kept for the next build; held by one building thread at a time
+    // (ilm::BuildWorkspace), given back when an allocation fails and with the
+    // context
+    void* build_ws = nullptr;
+    size_t build_bytes = 0;
+    std::atomic<bool> build_held{false};
     int trace_refill = 24;  // idle lanes of a wave that trigger its ray refill
     std::mutex mu;
 };
@@ -75,6 +83,20 @@ struct ilm_mesh {
 namespace ilm {
 // Ensures ctx->spill holds at least `words` 32-bit words.
 int ensure_spill(ilm_ctx* ctx, size_t words);
+// Holds ctx->build_ws for a scope, if it is wanted and no other thread does.
+struct BuildWorkspace {
+    ilm_ctx* ctx;
+    bool mine;
+    BuildWorkspace(ilm_ctx* c, bool want) : ctx(c), mine(want && !c->build_held.exchange(true)) {}
+    ~BuildWorkspace() {
+        if (mine) ctx->build_held.store(false);
+    }
+    BuildWorkspace(const BuildWorkspace&) = delete;
+    BuildWorkspace& operator=(const BuildWorkspace&) = delete;
+};
+// Ensures ctx->build_ws holds at least `bytes`; the caller holds it.
+constexpr size_t kBuildKeep = size_t(1) << 30;
+int ensure_build_ws(ilm_ctx* ctx, size_t bytes);
 // Takes this device's address of the fixed scratch of ilm_trace_closest_noalloc
 // and zeroes its fetch counters (once per device; called at context creation).
 int noalloc_setup(int device, hipStream_t stream);

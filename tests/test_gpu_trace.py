@@ -385,6 +385,32 @@ def test_lbvh_boxes_are_tight(ntri, gpu_ctx, ilm):
     m.close()
 
 
+@pytest.mark.parametrize("node_format", [0, 1])
+def test_lbvh_builds_reuse_the_workspace(node_format, gpu_ctx, ilm):
+    """Builds of growing and shrinking sizes, whose scratch is kept between
+    them, leave every mesh's own tree intact: hits equal the SAH tree's."""
+    built = []
+    for ntri in (3000, 60000, 2, 500, 60001):
+        pos, idx = meshgen.random_triangles(ntri, seed=ntri, extent=2.0, size=0.05)
+        m = ilm.Mesh(gpu_ctx, pos, idx)
+        m.build(builder=ilm.ILM_BUILDER_LBVH, node_format=node_format)
+        built.append((pos, idx, m))
+    for pos, idx, m in built:
+        ref = ilm.Mesh(gpu_ctx, pos, idx)
+        ref.build(node_format=node_format)
+        rays = meshgen.rays_toward(3000, pos, seed=2)
+        rb, ha, hb = ilm.rays_to_device(gpu_ctx, rays), gpu_ctx.buffer(3000 * 16), gpu_ctx.buffer(3000 * 16)
+        m.trace_closest(rb, 3000, ha)
+        ref.trace_closest(rb, 3000, hb)
+        gpu_ctx.sync()
+        a, b = ha.download(ilm.HIT_DTYPE, 3000), hb.download(ilm.HIT_DTYPE, 3000)
+        assert _compare_closest(a["prim"], a["t"], b["prim"], b["t"], f"lbvh {len(idx)}") >= 0.9999
+        for x in (rb, ha, hb):
+            x.free()
+        ref.close()
+        m.close()
+
+
 @pytest.mark.parametrize("kind", ["primary", "incoherent"])
 def test_c2_closest_matches_oracle_bvhmesh(c2, c2_oracle, gpu_ctx, ilm, orc, kind):
     """1,334,720 triangles: GPU closest hit vs the oracle's BVHMesh (reference
