@@ -19,8 +19,8 @@
 // the next layer takes D tiles 2c and 2c+1, i.e. K slot 8g+e of chunk c holds
 // feature perm(c,g,e) = 16(2c + e/4) + 4g + e%4; the packed weights use the
 // same K order. The backward pass chains the same way with W^T. Weight
-// gradients dW = G H^T reduce over samples in a separate kernel that reads
-// activations and gradients stored feature-major.
+// gradients dW = G H^T reduce over the samples of a workgroup in registers
+// (k_train) and over the workgroups in the optimiser (k_adam).
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
@@ -42,6 +42,8 @@ typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) short i16x2;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
 
 // Two floats rounded to bf16 (nearest even) by one v_cvt_pk_bf16_f32; wider
 // conversions compile to one conversion per value and a pack per pair.
@@ -193,16 +195,13 @@ __device__ __forceinline__ bf16x8 relu_pack(f32x4 a, f32x4 b) {
 __device__ __forceinline__ void order_after(int& off, float dep) { asm volatile("" : "+v"(off) : "v"(dep)); }
 
 // Copies `elems` bf16 (a multiple of 8) from global memory to LDS with the
-// whole workgroup. Each thread issues B loads of 16 B, then an empty asm
+// whole workgroup. Each thread issues six loads of 16 B, then an empty asm
 // statement takes every loaded value (so the compiler cannot move each load
 // down to its store), then the LDS stores follow. Copied one at a time, every
-// load waited for memory before its store: 39 round trips per thread for the
-// 80 KB of training weights (batched, the training kernel takes 6-8% less).
-// B = 6 covers the inference weights with 512 threads in one batch without
-// raising the kernel's registers.
-template <int B>
+// load waits for memory before its store. Six cover the inference weights
+// with 512 threads in one batch without raising the kernel's registers.
 __device__ __forceinline__ void lds_copy(__bf16* dst, const __bf16* src, int elems) {
-    static_assert(B == 6 || B == 16, "the asm statement below lists 6 or 16 values");
+    constexpr int B = 6;
     const u32x4* s = reinterpret_cast<const u32x4*>(src);
     u32x4* d = reinterpret_cast<u32x4*>(dst);
     const int n16 = elems / 8, nt = (int)blockDim.x;
@@ -211,12 +210,7 @@ __device__ __forceinline__ void lds_copy(__bf16* dst, const __bf16* src, int ele
         // past the end a lane re-reads the last element (its store is skipped)
 #pragma unroll
         for (int u = 0; u < B; ++u) v[u] = s[min(k0 + u * nt, n16 - 1)];
-        if constexpr (B == 6) {
-            asm volatile("" ::"v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]));
-        } else {
-            asm volatile("" ::"v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]),
-                         "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]), "v"(v[13]), "v"(v[14]), "v"(v[15]));
-        }
+        asm volatile("" ::"v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]));
 #pragma unroll
         for (int u = 0; u < B; ++u)
             if (k0 + u * nt < n16) d[k0 + u * nt] = v[u];
@@ -243,7 +237,7 @@ constexpr int kInferWaves = 8;
 
 __global__ void __launch_bounds__(64 * kInferWaves, 6) k_infer(InferArgs a) {
     __shared__ __bf16 w[kFwdElems];
-    lds_copy<6>(w, a.fwd, kFwdElems);
+    lds_copy(w, a.fwd, kFwdElems);
     __syncthreads();
     const int lane = (int)__lane_id(), g = lane >> 4, m = lane & 15;
     const int wave = threadIdx.x >> 6;
@@ -302,7 +296,33 @@ __global__ void __launch_bounds__(64 * kInferWaves, 6) k_infer(InferArgs a) {
     }
 }
 
-// ------------------------------------------------------------------ training: forward + backward
+// ------------------------------------------------------------------ training: gradients
+// Forward, backward and weight gradients in one kernel. A workgroup of eight
+// waves takes 128 samples at a time (16 per wave) and keeps its sum of every
+// weight gradient in registers: 92 output tiles of 16x16, 11 or 12 per wave.
+//
+// The products of a layer are computed twice with their operands exchanged,
+// which needs no other registers (a fragment of W is both A[out][in] and
+// B[in][out]): W H gives the next layer's operand (a lane holds features of
+// one sample), H^T W^T gives a lane four samples of one feature, the order in
+// which the weight gradient's reduction over samples reads them. The latter
+// are staged in LDS layer by layer of the backward pass (G_{l+1} and H_l,
+// feature-major), one barrier per layer with two buffers in turn, and each
+// wave adds its tiles of dW_l = G_{l+1} H_l^T. The network's input is
+// transposed by products with the identity, which are exact.
+//
+// Before, one kernel stored all activations and gradients for a second one
+// (98 MB written and read back per 65,536 samples). Steps of 65,536 samples,
+// Adam included, 61.4 -> 36.5 us; 4,096 samples 29.4 -> 17.1 us; 262,144 312
+// -> 81 us. What bounds it: 7.4 us per 128 samples and CU, a chain of layers
+// with one workgroup per CU (160 KB of LDS) whose LDS serves the weights'
+// fragments, the staging and the reductions (~11,000 of the 18,000 cycles);
+// and the workgroups' sums, 94 KB each, 10 us to write for 256 of them.
+constexpr int kTrainWaves = 8;
+constexpr int kTrainSamples = 16 * kTrainWaves;
+constexpr int kStageRow = kTrainSamples + 8;  // bf16 per staged feature: 272 bytes keep 16-byte reads of 16 rows conflict-free
+constexpr int kStageA = 2 * kHid, kStageB = kHid + kIn;  // features of the two buffers (layer 0 uses the second)
+
 struct TrainArgs {
     const __bf16* fwd;
     const __bf16* bwd;
@@ -310,93 +330,136 @@ struct TrainArgs {
     const float* targets;  // 4 floats per sample (rgb, weight)
     int64_t n;
     Bounds bd;
-    __bf16* H;  // activations, feature-major: H0 [96][n] then H1..H5 [64][n]
-    __bf16* G;  // gradients, feature-major: G1..G5 [64][n] then G6 [16][n]
-    int64_t ld;  // leading dimension of H and G (n rounded up to 32)
-    float* loss;  // per-sample loss (may be null)
+    float* loss;       // per-sample loss (may be null)
     float grad_scale;  // 1 / (3 n)
+    float* partial;    // [workgroups][kParams]
 };
 
-// One bf16 store at a row pointer plus a 32-bit byte offset.
-__device__ __forceinline__ void st_bf16(__bf16* row, uint32_t byte_off, __bf16 v) {
-    *reinterpret_cast<__bf16*>(reinterpret_cast<char*>(row) + byte_off) = v;
+// Four samples of one feature, rounded, from a transposed product.
+__device__ __forceinline__ bf16x4 relu_samples(f32x4 v) {
+    const u32x2 u = {relu_pair(v[0], v[1]), relu_pair(v[2], v[3])};
+    return __builtin_bit_cast(bf16x4, u);
 }
-__device__ __forceinline__ int64_t hoff(int layer, int64_t ld) { return layer == 0 ? 0 : (int64_t)kIn * ld + (int64_t)(layer - 1) * kHid * ld; }
-__device__ __forceinline__ int64_t goff(int layer, int64_t ld) { return (int64_t)(layer - 1) * kHid * ld; }  // layer 1..6
 
-// Two 256-thread workgroups per CU (80 KB of packed weights each in LDS).
-// 1024-thread workgroups (4 waves per SIMD) measured no faster: the kernel's
-// time goes to its feature-major activation and gradient stores.
-constexpr int kFbBlock = 256;
-__global__ void __launch_bounds__(kFbBlock) k_train_fb(TrainArgs a) {
+// Adds N tiles (rows: features 16 to.. of G; columns: features 16 ti.. of H)
+// over the staged samples.
+template <int N>
+__device__ __forceinline__ void add_tiles(f32x4 (&acc)[N], const __bf16* G, const __bf16* H, int to, int ti, int g,
+                                          int m) {
+#pragma unroll
+    for (int k = 0; k < kTrainSamples / 32; ++k) {
+        const bf16x8 A = *reinterpret_cast<const bf16x8*>(G + (16 * to + m) * kStageRow + 32 * k + 8 * g);
+#pragma unroll
+        for (int t = 0; t < N; ++t)
+            acc[t] = mfma32(A, *reinterpret_cast<const bf16x8*>(H + (16 * (ti + t) + m) * kStageRow + 32 * k + 8 * g),
+                            acc[t]);
+    }
+}
+// Sums of the gradients are written tile by tile as the lanes hold them (16
+// bytes a lane, whole lines): value r of lane l of tile t at (t * 64 + l) * 4 + r.
+// Tiles: layer 0 (to * 6 + ti), layers 1..4 (to * 4 + ti each), layer 5 (ti).
+__host__ __device__ __forceinline__ int tile_of(int layer, int to, int ti) {
+    return layer == 0 ? to * 6 + ti : layer <= 4 ? 24 + (layer - 1) * 16 + to * 4 + ti : 88 + ti;
+}
+// The weight (layer, o, i) whose gradient is at place p of a partial sum, and
+// its place among the master weights.
+__device__ __forceinline__ int weight_at(int p, int& layer, int& o, int& i) {
+    const int t = p >> 8, l = (p >> 2) & 63;
+    layer = t < 24 ? 0 : t < 88 ? 1 + (t - 24) / 16 : 5;
+    const int k = layer == 0 ? t : layer <= 4 ? (t - 24) % 16 : t - 88, cols = layer == 0 ? 6 : 4;
+    o = 16 * (k / cols) + 4 * (l >> 4) + (p & 3);
+    i = 16 * (k % cols) + (l & 15);
+    return layer == 0 ? kW0 + o * kIn + i : layer <= 4 ? kWh + ((layer - 1) * kHid + o) * kHid + i : kW5 + o * kHid + i;
+}
+template <int N>
+__device__ __forceinline__ void store_tiles(const f32x4 (&acc)[N], float* part, int tile) {
+#pragma unroll
+    for (int t = 0; t < N; ++t) reinterpret_cast<f32x4*>(part)[(tile + t) * 64 + (int)__lane_id()] = acc[t];
+}
+
+// ReLU's derivative of 16 outputs kept in one register: bits k and 16 + k tell
+// whether the two halves of pair k (bf16, never below 0) are above 0.
+__device__ __forceinline__ unsigned positive_bits(unsigned pair) {
+    const u16x2 one = __builtin_elementwise_min(__builtin_bit_cast(u16x2, pair), (u16x2)(unsigned short)1);
+    return __builtin_bit_cast(unsigned, one);
+}
+__device__ __forceinline__ unsigned halves_mask(unsigned bits) {  // 0x0000 or 0xFFFF per half from its lowest bit
+    return __builtin_bit_cast(unsigned, (u16x2)(unsigned short)0 - __builtin_bit_cast(u16x2, bits));
+}
+
+__global__ void __launch_bounds__(64 * kTrainWaves) k_train(TrainArgs a) {
     __shared__ __bf16 wf[kFwdElems];
     __shared__ __bf16 wb[kBwdElems];
-    lds_copy<16>(wf, a.fwd, kFwdElems);
-    lds_copy<16>(wb, a.bwd, kBwdElems);
+    __shared__ __align__(16) __bf16 stage[(kStageA + kStageB) * kStageRow];
+    lds_copy(wf, a.fwd, kFwdElems);
+    lds_copy(wb, a.bwd, kBwdElems);
     __syncthreads();
     const int lane = (int)__lane_id(), g = lane >> 4, m = lane & 15;
     const int wave = threadIdx.x >> 6;
-    constexpr int kWaves = kFbBlock / 64;
-    const int64_t n = a.n, ld = a.ld;
-    const int64_t step = (int64_t)gridDim.x * kWaves * 16;
-    for (int64_t base = ((int64_t)blockIdx.x * kWaves + wave) * 16; base < n; base += step) {
+    const int64_t n = a.n;
+    const int at = 16 * wave + 4 * g;  // this lane's first staged sample of a transposed product
+    bf16x8 eye[2];
+    for (int j = 0; j < 2; ++j)
+        for (int e = 0; e < 8; ++e) eye[j][e] = (__bf16)(8 * g + e == 16 * j + m ? 1.f : 0.f);
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    // the wave's weight-gradient tiles: layer 0 three, layers 1..4 two each,
+    // layer 5 one (waves 0..3)
+    const int to = wave >> 1, half = wave & 1;
+    f32x4 dw0[3] = {zero, zero, zero}, dw[4][2] = {{zero, zero}, {zero, zero}, {zero, zero}, {zero, zero}},
+          dw5[1] = {zero};
+    for (int64_t base = (int64_t)blockIdx.x * kTrainSamples; base < n; base += (int64_t)gridDim.x * kTrainSamples) {
         int lo8 = lane * 8, lo4 = lane * 4;  // opaque offsets: weights stay in LDS (see k_infer)
         asm volatile("" : "+v"(lo8), "+v"(lo4));
-        const int64_t smp = base + m;
+        const int64_t smp = base + 16 * wave + m;
         const bool valid = smp < n;
         const int64_t sl = valid ? smp : n - 1;
         float q[kQuery], pn[3];
         load_query(a.queries, sl, a.bd, q, pn);
+        const float4 tg = reinterpret_cast<const float4*>(a.targets)[sl];
         bf16x8 x[3];
         lane_features(q, pn[0], pn[1], pn[2], g, x);
-        // Each store is a row pointer plus the lane's 32-bit byte offset (the
-        // lane's sample, shifted by its group's 4 or 8 features; below 2^32
-        // for n <= 2^26). Every lane stores, with no mask per store: a wave's
-        // columns (base .. base + 15) lie below ld, and the weight-gradient
-        // reduction reads only columns below n.
-        const uint32_t off4 = 2u * (uint32_t)(4 * g * ld + smp), off8 = 2u * (uint32_t)(8 * g * ld + smp);
-        for (int c = 0; c < 3; ++c)
-            for (int e = 0; e < 8; ++e) st_bf16(a.H + hoff(0, ld) + (int64_t)(32 * c + e) * ld, off8, x[c][e]);
-        // hc = the current layer's output, as B chunks. Each layer's output is
-        // stored (H_l, for the weight gradients) as soon as it exists, and
-        // the backward pass keeps only its ReLU derivative: bit 8c + e of
-        // relu_on[l] is set when feature (c, e) of H_l is positive. Holding
-        // the masks instead of the five layers' outputs saves ~40 registers.
-        bf16x8 hc[2];
-        uint32_t relu_on[6];
-        f32x4 acc[4];
-        for (int t = 0; t < 4; ++t) {
-            acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-            for (int c = 0; c < 3; ++c)
-                acc[t] = mfma32(*reinterpret_cast<const bf16x8*>(wf + kF0 + (t * 3 + c) * 512 + lo8), x[c], acc[t]);
+        bf16x4 ht0[6], ht[5][4];  // transposed H_0 and H_1 .. H_5: tile t's feature 16t + m, samples 4g ..
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+            const f32x4 v = mfma32(x[t / 2], eye[t % 2], zero);
+            const u32x2 u = {bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
+            ht0[t] = __builtin_bit_cast(bf16x4, u);
         }
+        // hc: the current layer's output as B (or A) chunks; relu_on[l - 1]:
+        // positive_bits of H_l's pairs
+        bf16x8 hc[2];
+        uint32_t relu_on[5];
 #pragma unroll
         for (int l = 1; l <= 5; ++l) {
-            if (l > 1) {
-                for (int t = 0; t < 4; ++t) {
-                    acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    for (int c = 0; c < 2; ++c)
-                        acc[t] = mfma32(*reinterpret_cast<const bf16x8*>(wf + kFh + (l - 2) * 8 * 512 + (t * 2 + c) * 512 + lo8),
-                                        hc[c], acc[t]);
+            f32x4 acc[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                f32x4 tr = zero;
+                acc[t] = zero;
+#pragma unroll
+                for (int c = 0; c < (l == 1 ? 3 : 2); ++c) {
+                    const bf16x8 W = *reinterpret_cast<const bf16x8*>(
+                        wf + (l == 1 ? kF0 + (t * 3 + c) * 512 : kFh + (l - 2) * 8 * 512 + (t * 2 + c) * 512) + lo8);
+                    const bf16x8 h = l == 1 ? x[c] : hc[c < 2 ? c : 0];
+                    acc[t] = mfma32(W, h, acc[t]);
+                    tr = mfma32(h, W, tr);
                 }
+                ht[l - 1][t] = relu_samples(tr);
             }
-            for (int c = 0; c < 2; ++c) hc[c] = relu_pack(acc[2 * c], acc[2 * c + 1]);
-            order_after(lo8, acc[3][3]);
-            // store H_l (feature of K slot (c, g, e) is perm(c, g, e))
             uint32_t on = 0;
-            for (int c = 0; c < 2; ++c)
-                for (int e = 0; e < 8; ++e) {
-                    st_bf16(a.H + hoff(l, ld) + (int64_t)perm(c, 0, e) * ld, off4, hc[c][e]);
-                    on |= ((float)hc[c][e] > 0.f ? 1u : 0u) << (8 * c + e);
-                }
-            relu_on[l] = on;
+            for (int c = 0; c < 2; ++c) {
+                hc[c] = relu_pack(acc[2 * c], acc[2 * c + 1]);
+                const u32x4 u = __builtin_bit_cast(u32x4, hc[c]);
+                for (int k = 0; k < 4; ++k) on |= positive_bits(u[k]) << (4 * c + k);
+            }
+            relu_on[l - 1] = on;
+            order_after(lo8, acc[3][3]);
         }
-        f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+        f32x4 o = zero;
         for (int c = 0; c < 2; ++c) o = mfma32(*reinterpret_cast<const bf16x8*>(wf + kF5 + c * 512 + lo8), hc[c], o);
         // relative L2 loss on rgb: (y - t)^2 / (sg(y)^2 + 0.01); lanes g == 0 hold outputs 0..3
         bf16x4 g6;
         float lsum = 0.f;
-        float4 tg = reinterpret_cast<const float4*>(a.targets)[sl];
         for (int r = 0; r < 4; ++r) {
             float gr = 0.f;
             if (g == 0 && r < 3 && valid) {
@@ -408,129 +471,86 @@ __global__ void __launch_bounds__(kFbBlock) k_train_fb(TrainArgs a) {
             g6[r] = (__bf16)gr;
         }
         if (a.loss && g == 0 && valid) a.loss[smp] = lsum;
-        for (int r = 0; r < 4; ++r) st_bf16(a.G + goff(6, ld) + (int64_t)r * ld, off4, g6[r]);
-        // backward through layer 5 (x16 fragments): dH5 = W5^T g6
-        f32x4 d[4];
+        // layer 5: G_6 (its first four rows; the others are 0) and H_5
+        {
+            __bf16* G = stage;
+            __bf16* H = stage + kHid * kStageRow;
+            if (g == 0)
+                for (int r = 0; r < 4; ++r) G[r * kStageRow + 16 * wave + m] = g6[r];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) *reinterpret_cast<bf16x4*>(H + (16 * t + m) * kStageRow + at) = ht[4][t];
+            __syncthreads();
+            if (wave < 4) {
+#pragma unroll
+                for (int k = 0; k < kTrainSamples / 32; ++k) {
+                    bf16x8 A = *reinterpret_cast<const bf16x8*>(G + (m & 3) * kStageRow + 32 * k + 8 * g);
+                    if (m >= 4) A = bf16x8{};
+                    dw5[0] = mfma32(A, *reinterpret_cast<const bf16x8*>(H + (16 * wave + m) * kStageRow + 32 * k + 8 * g),
+                                    dw5[0]);
+                }
+            }
+        }
+        // backward through layer 5 (x16 fragments): dH5 = W5^T g6, and transposed
+        f32x4 d[4], dt[4];
         order_after(lo4, (float)g6[0]);
-        for (int t = 0; t < 4; ++t)
-            d[t] = mfma16(*reinterpret_cast<const bf16x4*>(wb + kB5 + t * 256 + lo4), g6, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const bf16x4 W = *reinterpret_cast<const bf16x4*>(wb + kB5 + t * 256 + lo4);
+            d[t] = mfma16(W, g6, zero);
+            dt[t] = mfma16(g6, W, zero);
+        }
 #pragma unroll
         for (int l = 5; l >= 1; --l) {
-            // G_l = dH_l * relu'(H_l), back in B-chunk form
-            bf16x8 gl[2];
-            for (int c = 0; c < 2; ++c) {
-                float v[8];
-                for (int e = 0; e < 8; ++e) v[e] = ((relu_on[l] >> (8 * c + e)) & 1u) ? d[2 * c + (e >> 2)][e & 3] : 0.f;
-                const u32x4 u = {bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3]), bf16_pair(v[4], v[5]), bf16_pair(v[6], v[7])};
-                gl[c] = __builtin_bit_cast(bf16x8, u);
-            }
-            for (int c = 0; c < 2; ++c)
-                for (int e = 0; e < 8; ++e) st_bf16(a.G + goff(l, ld) + (int64_t)perm(c, 0, e) * ld, off4, gl[c][e]);
-            if (l == 1) break;
-            order_after(lo8, d[3][3]);
-            // dH_{l-1} = W_{l-1}^T G_l  (layer index of the weights is l-1, 1..4)
+            // G_l = dH_l * relu'(H_l): in B-chunk form, and staged with H_{l-1}
+            __bf16* G = stage + (l & 1 ? kStageA * kStageRow : 0);
+            __bf16* H = G + kHid * kStageRow;
+#pragma unroll
             for (int t = 0; t < 4; ++t) {
-                d[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                for (int c = 0; c < 2; ++c)
-                    d[t] = mfma32(*reinterpret_cast<const bf16x8*>(wb + kBh + (l - 2) * 8 * 512 + (t * 2 + c) * 512 + lo8),
-                                  gl[c], d[t]);
+                const u32x2 h = __builtin_bit_cast(u32x2, ht[l - 1][t]);
+                const u32x2 u = {bf16_pair(dt[t][0], dt[t][1]) & halves_mask(positive_bits(h[0])),
+                                 bf16_pair(dt[t][2], dt[t][3]) & halves_mask(positive_bits(h[1]))};
+                *reinterpret_cast<u32x2*>(G + (16 * t + m) * kStageRow + at) = u;
             }
-        }
-    }
-}
-
-// ------------------------------------------------------------------ weight gradients
-// 92 output tiles of 16x16 in 21 strips of tiles sharing their output rows:
-// layer 0 (4 strips of 6 tiles), layers 1..4 (4 strips of 4 tiles each),
-// layer 5 (1 strip of 4 tiles). A wave computes one strip over its
-// workgroup's chunk of samples, so the strip's G rows are read once for all
-// of its tiles.
-constexpr int kStrips = 21;
-constexpr int kStripWaves = 24;  // six workgroups of four waves per chunk
-struct DwArgs {
-    const __bf16* H;
-    const __bf16* G;
-    int64_t n;         // samples
-    int64_t ld;        // leading dimension of H and G (multiple of 32)
-    int64_t chunk;     // samples per block (multiple of 32)
-    float* partial;    // [blocks][kParams]
-};
-
-__device__ __forceinline__ void strip_of(int strip, int& layer, int& to, int& ntiles) {
-    if (strip < 4) { layer = 0; to = strip; ntiles = 6; return; }
-    if (strip < 20) { layer = 1 + (strip - 4) / 4; to = (strip - 4) % 4; ntiles = 4; return; }
-    layer = 5; to = 0; ntiles = 4;
-}
-
-__global__ void __launch_bounds__(256, 3) k_dw(DwArgs a) {
-    const int lane = (int)__lane_id(), g = lane >> 4, m = lane & 15;
-    const int wave = threadIdx.x >> 6;
-    const int strip = (int)blockIdx.y * 4 + wave;
-    if (strip >= kStrips) return;
-    const int64_t n = a.n, ld = a.ld;
-    const int64_t s0 = (int64_t)blockIdx.x * a.chunk, s1 = min(n, s0 + a.chunk);
-    float* part = a.partial + (int64_t)blockIdx.x * kParams;
-    int layer, to, ntiles;
-    strip_of(strip, layer, to, ntiles);
-    // A rows: G_{layer+1} output features; B rows: H_layer input features
-    const __bf16* gA = a.G + (int64_t)layer * kHid * ld + (int64_t)(16 * to + m) * ld;
-    const __bf16* hB = a.H + (layer == 0 ? 0 : (int64_t)kIn * ld + (int64_t)(layer - 1) * kHid * ld) + (int64_t)m * ld;
-    f32x4 acc[6];
 #pragma unroll
-    for (int t = 0; t < 6; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // Three steps of 32 samples at a time: their loads are all issued before
-    // the first product, so a wave waits for memory once per 96 samples (four
-    // steps need more than the 168 registers of three waves per SIMD).
-    constexpr int kSteps = 3;
-    int64_t s = s0;
-    for (; s + 32 * kSteps <= s1; s += 32 * kSteps) {
-        bf16x8 A[kSteps], B[kSteps][6];
+            for (int t = 0; t < (l == 1 ? 6 : 4); ++t)
+                *reinterpret_cast<bf16x4*>(H + (16 * t + m) * kStageRow + at) = l == 1 ? ht0[t] : ht[l == 1 ? 0 : l - 2][t < 4 ? t : 0];
+            bf16x8 gl[2];
+            if (l > 1) {
+                for (int c = 0; c < 2; ++c) {
+                    u32x4 u;
+                    for (int k = 0; k < 4; ++k) {
+                        const f32x4 v = d[2 * c + (k >> 1)];
+                        u[k] = bf16_pair(v[2 * (k & 1)], v[2 * (k & 1) + 1]) &
+                               halves_mask(relu_on[l - 1] >> (4 * c + k) & 0x00010001u);
+                    }
+                    gl[c] = __builtin_bit_cast(bf16x8, u);
+                }
+                order_after(lo8, d[3][3]);
+            }
+            __syncthreads();
+            if (l > 1) {
+                add_tiles(dw[l - 2], G, H, to, 2 * half, g, m);
+                // dH_{l-1} = W_{l-1}^T G_l (layer index of the weights is l-1, 1..4)
 #pragma unroll
-        for (int u = 0; u < kSteps; ++u) {
-            const int64_t k0 = s + 32 * u + 8 * g;
-            A[u] = *reinterpret_cast<const bf16x8*>(gA + k0);
+                for (int t = 0; t < 4; ++t) {
+                    d[t] = dt[t] = zero;
 #pragma unroll
-            for (int t = 0; t < 6; ++t)
-                if (t < ntiles) B[u][t] = *reinterpret_cast<const bf16x8*>(hB + (int64_t)(16 * t) * ld + k0);
-        }
-#pragma unroll
-        for (int u = 0; u < kSteps; ++u)
-#pragma unroll
-            for (int t = 0; t < 6; ++t)
-                if (t < ntiles) acc[t] = mfma32(A[u], B[u][t], acc[t]);
-    }
-    for (; s < s1; s += 32) {
-        const int64_t k0 = s + 8 * g;
-        const bool full = k0 + 8 <= s1;
-        bf16x8 A;
-        if (full) {
-            A = *reinterpret_cast<const bf16x8*>(gA + k0);
-        } else {
-            for (int e = 0; e < 8; ++e) A[e] = k0 + e < s1 ? gA[k0 + e] : (__bf16)0.f;
-        }
-#pragma unroll
-        for (int t = 0; t < 6; ++t) {
-            if (t >= ntiles) break;
-            const __bf16* hp = hB + (int64_t)(16 * t) * ld;
-            bf16x8 B;
-            if (full) {
-                B = *reinterpret_cast<const bf16x8*>(hp + k0);
+                    for (int c = 0; c < 2; ++c) {
+                        const bf16x8 W = *reinterpret_cast<const bf16x8*>(wb + kBh + (l - 2) * 8 * 512 + (t * 2 + c) * 512 + lo8);
+                        if (l > 2) d[t] = mfma32(W, gl[c], d[t]);  // G_1 is needed transposed only
+                        dt[t] = mfma32(gl[c], W, dt[t]);
+                    }
+                }
             } else {
-                for (int e = 0; e < 8; ++e) B[e] = k0 + e < s1 ? hp[k0 + e] : (__bf16)0.f;
+                add_tiles(dw0, G, H, to, 3 * half, g, m);
             }
-            acc[t] = mfma32(A, B, acc[t]);
         }
     }
-    const int in_dim = layer == 0 ? kIn : kHid;
-    const int base = layer == 0 ? kW0 : (layer <= 4 ? kWh + (layer - 1) * kHid * kHid : kW5);
+    float* part = a.partial + (int64_t)blockIdx.x * kParams;
+    store_tiles(dw0, part, tile_of(0, to, 3 * half));
 #pragma unroll
-    for (int t = 0; t < 6; ++t) {
-        if (t >= ntiles) break;
-        for (int r = 0; r < 4; ++r) {
-            const int o = 16 * to + 4 * g + r, i = 16 * t + m;
-            part[base + o * in_dim + i] = acc[t][r];
-        }
-    }
+    for (int l = 0; l < 4; ++l) store_tiles(dw[l], part, tile_of(1 + l, to, 2 * half));
+    if (wave < 4) store_tiles(dw5, part, tile_of(5, 0, wave));
 }
 
 // ------------------------------------------------------------------ Adam + repack
@@ -547,39 +567,43 @@ struct AdamArgs {
     int do_update;
 };
 
-// 64 parameters per workgroup: its four waves sum every fourth sample
-// chunk's partial gradients (a fixed order, so the sum is deterministic),
-// the first wave adds the four sums and updates.
-__global__ void __launch_bounds__(256) k_adam(AdamArgs a) {
-    __shared__ float quarter[4][64];
+// 64 weights per workgroup, in the partial sums' order: its waves sum every
+// kAdamWaves-th partial gradient (a fixed order, so the sum is deterministic),
+// the first wave adds the waves' sums in order and updates. 6 us for 256
+// partials (24 MB, about the time a copy takes to read them).
+constexpr int kAdamWaves = 8;
+__global__ void __launch_bounds__(64 * kAdamWaves) k_adam(AdamArgs a) {
+    __shared__ float sums[kAdamWaves][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int p = blockIdx.x * 64 + lane;
     float part = 0.f;
-    if (a.do_update && p < kParams) {
-        // eight rows in flight per wave (independent loads; the sum keeps its order)
-#pragma unroll 8
-        for (int b = wave; b < a.nblocks; b += 4) part += a.partial[(int64_t)b * kParams + p];
-    }
-    quarter[wave][lane] = part;
-    __syncthreads();
-    if (wave != 0 || p >= kParams) return;
-    float wv = a.w[p];
     if (a.do_update) {
-        const float gsum = (quarter[0][lane] + quarter[1][lane]) + (quarter[2][lane] + quarter[3][lane]);
-        a.grad[p] = gsum;
-        float m1 = a.b1 * a.mom1[p] + (1.f - a.b1) * gsum;
-        float m2 = a.b2 * a.mom2[p] + (1.f - a.b2) * gsum * gsum;
-        a.mom1[p] = m1;
-        a.mom2[p] = m2;
-        wv -= a.lr * (m1 / a.c1) / (sqrtf(m2 / a.c2) + a.eps);
-        a.w[p] = wv;
+        // sixteen rows in flight per wave (independent loads; the sum keeps its order)
+#pragma unroll 16
+        for (int b = wave; b < a.nblocks; b += kAdamWaves) part += a.partial[(int64_t)b * kParams + p];
     }
-    int o, i;
-    int layer = layer_of(p, o, i);
+    sums[wave][lane] = part;
+    __syncthreads();
+    if (wave != 0) return;
+    int layer, o, i;
+    const int at = weight_at(p, layer, o, i);
+    float wv = a.w[at];
+    if (a.do_update) {
+        float gsum = sums[0][lane];
+        for (int k = 1; k < kAdamWaves; ++k) gsum += sums[k][lane];
+        a.grad[at] = gsum;
+        float m1 = a.b1 * a.mom1[at] + (1.f - a.b1) * gsum;
+        float m2 = a.b2 * a.mom2[at] + (1.f - a.b2) * gsum * gsum;
+        a.mom1[at] = m1;
+        a.mom2[at] = m2;
+        wv -= a.lr * (m1 / a.c1) / (sqrtf(m2 / a.c2) + a.eps);
+        a.w[at] = wv;
+    }
     __bf16 b = (__bf16)wv;
     a.fwd[fwd_pos(layer, o, i)] = b;
     if (layer >= 1) a.bwd[bwd_pos(layer, o, i)] = b;
 }
+static_assert(kParams % 64 == 0, "k_adam covers whole groups of 64 weights");
 
 // ------------------------------------------------------------------ layout self-test
 // D = A B for one 16x16x32 and one 16x16x16 product with integer-valued
@@ -621,9 +645,6 @@ struct ilm_nrc {
     __bf16* fwd = nullptr;
     __bf16* bwd = nullptr;
     // training scratch, grown on demand
-    int64_t cap = 0;
-    __bf16* H = nullptr;
-    __bf16* G = nullptr;
     float* partial = nullptr;
     int64_t partial_blocks = 0;
 };
@@ -673,7 +694,7 @@ int nrc_repack(ilm_nrc* r, hipStream_t st, int update, float c1, float c2, int n
     a.c1 = c1;
     a.c2 = c2;
     a.do_update = update;
-    hipLaunchKernelGGL(k_adam, dim3((kParams + 63) / 64), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_adam, dim3(kParams / 64), dim3(64 * kAdamWaves), 0, st, a);
     return hipGetLastError() == hipSuccess ? ILM_OK : ilm::fail(ILM_ERR_HIP, "adam launch");
 }
 
@@ -701,25 +722,14 @@ int layout_selftest(ilm_ctx* ctx) {
     return ILM_OK;
 }
 
-int ensure_train(ilm_nrc* r, int64_t n, int64_t blocks) {
-    n = (n + 31) / 32 * 32;
-    if (r->cap < n) {
-        if (r->H) ilm_free(r->ctx, r->H);
-        if (r->G) ilm_free(r->ctx, r->G);
-        r->H = r->G = nullptr;
-        r->cap = 0;
-        int rc = ilm_alloc(r->ctx, (size_t)n * (kIn + 5 * kHid) * 2, (void**)&r->H);
-        if (!rc) rc = ilm_alloc(r->ctx, (size_t)n * (5 * kHid + kOut) * 2, (void**)&r->G);
-        if (rc) return rc;
-        r->cap = n;
-    }
-    if (r->partial_blocks < blocks) {
-        if (r->partial) ilm_free(r->ctx, r->partial);
-        r->partial = nullptr;
-        int rc = ilm_alloc(r->ctx, (size_t)blocks * kParams * 4, (void**)&r->partial);
-        if (rc) return rc;
-        r->partial_blocks = blocks;
-    }
+int ensure_train(ilm_nrc* r, int64_t blocks) {
+    if (r->partial_blocks >= blocks) return ILM_OK;
+    if (r->partial) ilm_free(r->ctx, r->partial);
+    r->partial = nullptr;
+    r->partial_blocks = 0;
+    int rc = ilm_alloc(r->ctx, (size_t)blocks * kParams * 4, (void**)&r->partial);
+    if (rc) return rc;
+    r->partial_blocks = blocks;
     return ILM_OK;
 }
 }  // namespace
@@ -781,8 +791,7 @@ int ilm_nrc_create(ilm_ctx* ctx, const ilm_nrc_params* p, ilm_nrc** out) {
 
 int ilm_nrc_destroy(ilm_nrc* r) {
     if (!r) return ILM_OK;
-    for (void* p : {(void*)r->w, (void*)r->m1, (void*)r->m2, (void*)r->grad, (void*)r->fwd, (void*)r->bwd, (void*)r->H, (void*)r->G,
-                    (void*)r->partial})
+    for (void* p : {(void*)r->w, (void*)r->m1, (void*)r->m2, (void*)r->grad, (void*)r->fwd, (void*)r->bwd, (void*)r->partial})
         if (p) ilm_free(r->ctx, p);
     delete r;
     return ILM_OK;
@@ -823,11 +832,10 @@ int ilm_nrc_infer(ilm_nrc* r, const float* queries, int64_t n, float* out, void*
 
 int ilm_nrc_train_step(ilm_nrc* r, const float* queries, const float* targets, int64_t n, float* loss, void* stream) {
     if (!r || n <= 0 || !queries || !targets) return ilm::fail(ILM_ERR_INVALID, "bad arguments");
-    // the training kernel addresses activations with 32-bit lane offsets
     if (n > (int64_t(1) << 26)) return ilm::fail(ILM_ERR_INVALID, "training batch above 2^26 samples");
-    const int64_t chunk = 512;
-    const int64_t dw_blocks = (n + chunk - 1) / chunk;
-    int rc = ensure_train(r, n, dw_blocks);
+    // one workgroup per CU (its LDS allows no more), fewer for small batches
+    const int64_t blocks = std::min<int64_t>((n + kTrainSamples - 1) / kTrainSamples, r->ctx->cu_count);
+    int rc = ensure_train(r, blocks);
     if (rc) return rc;
     hipStream_t st = ilm::pick_stream(r->ctx, stream);
     TrainArgs t;
@@ -837,27 +845,14 @@ int ilm_nrc_train_step(ilm_nrc* r, const float* queries, const float* targets, i
     t.targets = targets;
     t.n = n;
     t.bd = r->bd;
-    t.H = r->H;
-    t.G = r->G;
-    t.ld = (n + 31) / 32 * 32;
     t.loss = loss;
     t.grad_scale = 1.f / (3.f * (float)n);
-    const int64_t fb_per_block = kFbBlock / 64 * 16;  // 16 samples per wave
-    int64_t fb_blocks = std::min<int64_t>((n + fb_per_block - 1) / fb_per_block, (int64_t)r->ctx->cu_count * 2);
-    hipLaunchKernelGGL(k_train_fb, dim3((unsigned)fb_blocks), dim3(kFbBlock), 0, st, t);
-    DwArgs d;
-    d.H = r->H;
-    d.G = r->G;
-    d.n = n;
-    d.ld = (n + 31) / 32 * 32;
-    d.chunk = chunk;
-    d.partial = r->partial;
-    // six workgroups per chunk of samples, one wave per strip of output tiles
-    hipLaunchKernelGGL(k_dw, dim3((unsigned)dw_blocks, kStripWaves / 4), dim3(256), 0, st, d);
+    t.partial = r->partial;
+    hipLaunchKernelGGL(k_train, dim3((unsigned)blocks), dim3(64 * kTrainWaves), 0, st, t);
     ILM_HIP(hipGetLastError());
     r->step += 1;
     float c1 = 1.f - powf(r->b1, (float)r->step), c2 = 1.f - powf(r->b2, (float)r->step);
-    return nrc_repack(r, st, 1, c1, c2, (int)dw_blocks);
+    return nrc_repack(r, st, 1, c1, c2, (int)blocks);
 }
 
 }  // extern "C"

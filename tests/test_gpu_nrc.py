@@ -84,6 +84,50 @@ def test_gradients_and_adam_match_oracle(gpu_ctx, ilm):
     net.close()
 
 
+@pytest.mark.parametrize("n", [1, 15, 17, 127, 128, 129, 1000, 32769])
+def test_gradients_at_sample_counts_around_the_workgroups(gpu_ctx, ilm, n):
+    """Part of a wave's 16 samples, part of a workgroup's 128, one and two
+    rounds of workgroups, weights of 0 for some samples.
+
+    Against the oracle: inputs that differ by a rounding (the encoding's sines)
+    switch a hidden unit whose sum is within it of 0 on or off, in about one
+    sample of a hundred; one unit of 64 in one sample of n is 1 / sqrt(64 n)
+    of a layer's gradient norm (contributions of random signs); four such and
+    the 2e-2 of many samples are allowed.
+
+    Against itself: the samples moved behind as many of weight 0 (other lanes,
+    waves and workgroups, twice the count: every gradient exactly half) give
+    the same gradient up to the order of the sums, 1e-5."""
+    net = ilm.Nrc(gpu_ctx, LO, HI, lr=1e-3)
+    w = onrc.init_weights(9)
+    net.set_weights(w)
+    q = _queries(n, n)
+    rng = np.random.default_rng(n + 1)
+    t = np.zeros((n, 4), np.float32)
+    t[:, :3] = rng.uniform(0, 2, (n, 3))
+    t[:, 3] = rng.integers(0, 2, n) if n > 1 else 1
+    qb, tb, lb = gpu_ctx.to_device(q), gpu_ctx.to_device(t), gpu_ctx.buffer(n * 4)
+    net.train_step(qb, tb, n, lb)
+    gpu_ctx.sync()
+    g = net.gradients().astype(np.float64)
+    loss, go = onrc.loss_grad(w, onrc.encode(q, LO, HI), t, weight=t[:, 3], use_bf16=True)
+    gl = lb.download(np.float32, n)
+    assert abs(gl.sum() / (3 * n) - loss) <= 2e-3 * loss
+    off = 0
+    for k, (o, i) in enumerate(onrc.SHAPES):
+        s = slice(off, off + o * i)
+        assert _rel(g[s], go[s]) < 2e-2 + 4 / np.sqrt(64 * n), k
+        off += o * i
+    q2, t2 = gpu_ctx.to_device(np.concatenate([q, q])), gpu_ctx.to_device(np.concatenate([t * [1, 1, 1, 0], t]).astype(np.float32))
+    net.set_weights(w)
+    net.train_step(q2, t2, 2 * n)
+    gpu_ctx.sync()
+    assert _rel(2 * net.gradients().astype(np.float64), g) < 1e-5
+    for x in (qb, tb, lb, q2, t2):
+        x.free()
+    net.close()
+
+
 def test_training_fits_a_smooth_field(gpu_ctx, ilm):
     """Online training on a fixed synthetic radiance field lowers the loss and
     generalises to held-out queries."""
