@@ -32,6 +32,7 @@ namespace ilm {
 constexpr int kTraceSegs = 8;           // ray segments of a traversal launch (one per XCD)
 constexpr int kSegCounter0 = 64;        // first segment counter in ilm_ctx::counters
 constexpr int kSegCounterStride = 64;   // 512 bytes between segment counters
+constexpr int kSegDone = 16;            // a segment's counter of finished waves, 128 bytes after its ray counter
 constexpr int kCounterWords = kSegCounter0 + kTraceSegs * kSegCounterStride;
 }  // namespace ilm
 
@@ -45,7 +46,7 @@ struct ilm_ctx {
     int next_event = 0;
     // per-context scratch for traversal: ray-fetch counters and the
     // traversal-stack spill area, grown on demand
-    // [1] finished waves, [2] error flags, [4] post-process scratch; the
+    // [1] segments whose waves have finished, [2] error flags, [4] post-process scratch; the
     // ray-fetch counters of the kTraceSegs ray segments at
     // kSegCounter0 + k * kSegCounterStride (each on its own 512-byte line)
     unsigned long long* counters = nullptr;

@@ -9,8 +9,11 @@
 // blockIdx % 8, which under the round-robin dispatch of workgroups to the
 // eight XCDs is its XCD's own, and moves on once a segment is spent. Each
 // XCD's L2 then serves a narrow window of neighbouring (coherent) rays, and
-// the fetch atomics spread over eight counters. Only the first ceil(n / 64)
-// waves of the grid take part, so short launches stay cheap. A wave refills once at
+// the fetch atomics spread over eight counters. Atomics on one address are
+// served one after another at some 6 ns each, so those that all waves issue
+// at once are avoided: a wave's first rays are dealt to it, the waves of a
+// workgroup share what they find spent, and the end of a launch is counted
+// per XCD. Short launches deal out all their rays. A wave refills once at
 // least refill_min of its lanes are idle (24 by default; 56 for coherent
 // camera rays, whose lanes finish together). Per lane: a 16-entry
 // traversal stack ring in LDS (lane-strided, conflict-free) that spills its
@@ -45,6 +48,8 @@ namespace ilm {
 
 constexpr int kBlock = 256;
 constexpr int kLds = 16;
+// Waves per CU over which a short launch's rays are dealt out.
+constexpr int kShortWaves = 8;
 
 struct TraceArgs {
     const float4* __restrict__ nodes;  // wide nodes (Kind<K>::F4 float4 each)
@@ -62,6 +67,7 @@ struct TraceArgs {
     int64_t grid_threads;
     unsigned long long* counters;
     uint32_t total_waves;
+    uint32_t short_waves;
     // dual launches: a second queue traced for any hits in the same launch,
     // as ids n1 .. n1 + n2 of the combined range (n1 = the first queue's count)
     const ilm_ray* __restrict__ rays2;
@@ -224,27 +230,56 @@ __global__ void __launch_bounds__(kBlock, (kTraceWaves<KIND, STATS>)) k_trace4(T
     // per lane: a kLds-entry stack ring (lane-strided, conflict-free) and W
     // staging words for the current node's child words
     __shared__ __align__(16) uint32_t lds[(kLds + W) * kBlock];
+    __shared__ uint32_t s_spent;  // the most segments a wave of the workgroup has found spent (long launches)
     const int tid = threadIdx.x;
     uint32_t* const ring = lds + tid;
     uint32_t* const stage = lds + kLds * kBlock + tid * W;
     const uint32_t stage_off = (uint32_t)((kLds * kBlock + tid * W) * sizeof(uint32_t));
-    const int64_t gtid = (int64_t)blockIdx.x * kBlock + tid;
-    const int64_t n1 = a.n_dev ? (int64_t)min((unsigned long long)a.n, *a.n_dev) : a.n;
-    const int64_t n = DUAL ? n1 + (a.n2_dev ? (int64_t)min((unsigned long long)a.n2, *a.n2_dev) : a.n2) : n1;
-    // only the first ceil(n / 64) waves can receive rays: the others leave at
-    // once, without touching the counters, so that a short launch (the late
-    // bounces of a frame) costs few atomics
-    const unsigned long long wave_id = (unsigned long long)gtid >> 6;
-    const unsigned long long part = min((unsigned long long)a.total_waves, ((unsigned long long)n + 63ull) >> 6);
-    if (wave_id >= part) return;
-    const unsigned long long seg_len = ((unsigned long long)n + kTraceSegs - 1) / kTraceSegs;
+    const uint32_t gtid = blockIdx.x * kBlock + (uint32_t)tid;
+    // launches hold fewer than 2^32 rays (checked on the host)
+    const uint32_t n1 = a.n_dev ? (uint32_t)min((unsigned long long)a.n, *a.n_dev) : (uint32_t)a.n;
+    const uint32_t n = DUAL ? n1 + (a.n2_dev ? (uint32_t)min((unsigned long long)a.n2, *a.n2_dev) : (uint32_t)a.n2) : n1;
+    // Every wave's first rays are dealt to it, without an atomic: in a short
+    // launch (at most 64 rays per wave of the grid) all there are, in equal
+    // shares to at most short_waves waves or, when those are full, 64 to each;
+    // in a long one the first rays of its XCD's segment. Short shares are
+    // dealt to the XCDs in contiguous runs, as the segments are, among the
+    // workgroups that get any. A wave's instructions cost the same however
+    // few of its lanes hold rays, so fewer rays per wave pay only while the
+    // vector ALUs idle: two waves per SIMD (kShortWaves = 8 per CU; 4, 12 and
+    // 16 within 4%, and seven per SIMD 10% slower at 100,000 rays).
+    // Incoherent rays, 1.33M triangles, fetched before and dealt out now:
+    // 1,600 rays 97 -> 61 us, 40,000 142 -> 109, 202,500 178 -> 164, 448,900
+    // 272 -> 229; 1,000 rays among 2,048 instances 438 -> 110; 1,000 in the
+    // 42-triangle room 17.5 -> 9.3. Long launches: 1M rays 391 -> 331 us (of
+    // which the dealt first rays 20, the shared ends of segments 30, the
+    // count per XCD 6), 4.2M 930 -> 867.
+    const bool shared_out = n <= a.total_waves * 64u;
+    const uint32_t seg_len = n / kTraceSegs + (n % kTraceSegs ? 1u : 0u);
+    const uint32_t xcd = blockIdx.x % kTraceSegs, wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid / 64);
+    uint32_t own, end;  // the wave's share [own, end), at most a ray per lane
+    if (shared_out) {
+        const uint32_t per = min((n + a.short_waves - 1u) / a.short_waves, 64u);
+        const uint32_t busy = n ? (n + per - 1u) / per : 0u;
+        const uint32_t blocks = (busy + kBlock / 64 - 1) / (kBlock / 64);
+        if (blockIdx.x >= blocks) return;
+        const uint32_t block = xcd * (blocks / kTraceSegs) + min(xcd, blocks % kTraceSegs) + blockIdx.x / kTraceSegs;
+        own = (block * (kBlock / 64) + wave) * per;
+        if (own >= n) return;
+        end = min(own + per, n);
+    } else {
+        own = xcd * seg_len + (blockIdx.x / kTraceSegs * (kBlock / 64) + wave) * 64u;
+        end = min(own + 64u, xcd * seg_len + min(seg_len, n - min(xcd * seg_len, n)));
+        if (tid == 0) s_spent = 0;
+        __syncthreads();
+    }
 
     bool active = false;
     bool exhausted = false;  // uniform across the wave
-    // the segment the wave fetches from (it starts on its XCD's) and the
-    // number of segments it has found spent; uniform across the wave
-    unsigned int seg = blockIdx.x % kTraceSegs, spent = 0;
-    uint32_t ray_id = 0;  // launches hold fewer than 2^32 rays (checked on the host)
+    // the segments from its XCD's on that the wave has found spent (it fetches
+    // from the next); uniform across the wave
+    unsigned int spent = 0;
+    uint32_t ray_id = 0;
     bool any_ray = ANY;  // this lane's ray wants any hit (dual launches: the second queue's rays)
     RayState r;
     uint32_t cur = kNoNode;
@@ -261,6 +296,12 @@ __global__ void __launch_bounds__(kBlock, (kTraceWaves<KIND, STATS>)) k_trace4(T
     bool world_stale = false;          // INST: r still holds an instance's object-space set-up
     int32_t inst_id = -1, best_inst = -1;
 
+    // rays of segment k, and how many of its first ones were dealt to the
+    // waves of its XCD (its counter counts from there)
+    auto seg_size = [&](uint32_t k) -> uint32_t { return min(seg_len, n - min(k * seg_len, n)); };
+    auto first_fetched = [&](uint32_t k) -> uint32_t {
+        return (gridDim.x + kTraceSegs - 1 - k) / kTraceSegs * kBlock;
+    };
     auto pop = [&]() -> uint32_t {
         if (sp > base) {
             --sp;
@@ -276,7 +317,7 @@ __global__ void __launch_bounds__(kBlock, (kTraceWaves<KIND, STATS>)) k_trace4(T
         if (ANY) {
             a.occ[ray_id] = best_prim >= 0 ? 1 : 0;
         } else if (DUAL && any_ray) {
-            a.occ2[ray_id - (uint32_t)n1] = best_prim >= 0 ? 1 : 0;
+            a.occ2[ray_id - n1] = best_prim >= 0 ? 1 : 0;
         } else {
             float4 h = make_float4(best_t, __int_as_float(best_prim), best_u, best_v);
             reinterpret_cast<float4*>(a.hits)[ray_id] = h;
@@ -315,33 +356,44 @@ __global__ void __launch_bounds__(kBlock, (kTraceWaves<KIND, STATS>)) k_trace4(T
         unsigned long long idle = __ballot(!active);
         if (!exhausted && idle != 0ull && (__popcll(idle) >= a.refill_min || idle == ~0ull)) {
             // idle lanes take the next ray ids of the current segment; a spent
-            // segment sends the wave on to the next one
-            const unsigned long long need = (unsigned long long)__popcll(idle);
-            const unsigned long long rank = (unsigned long long)__popcll(idle & __lanemask_lt());
-            unsigned long long got = 0, mine = ~0ull;
-            while (got < need && spent < (unsigned)kTraceSegs) {
-                const unsigned long long s0 = seg * seg_len;
-                const unsigned long long s1 = min(s0 + seg_len, (unsigned long long)n);
-                const unsigned long long size = s1 > s0 ? s1 - s0 : 0ull;
-                const unsigned long long want = need - got;
-                unsigned long long base = 0;
-                if (__lane_id() == 0) base = atomicAdd(&a.counters[kSegCounter0 + seg * kSegCounterStride], want);
-                base = __shfl(base, 0);
-                const unsigned long long take = base < size ? min(want, size - base) : 0ull;
-                if (rank >= got && rank < got + take) mine = s0 + base + (rank - got);
+            // segment sends the wave, and the others of its workgroup when
+            // they fetch next, on to the next one
+            const uint32_t need = (uint32_t)__popcll(idle), rank = (uint32_t)__popcll(idle & __lanemask_lt());
+            uint32_t got = 0, mine = 0;
+            bool given = false;
+            if (own != ~0u) {
+                given = own + rank < end;
+                mine = own + rank;
+                got = need;
+                own = ~0u;  // dealt
+                exhausted = shared_out;
+            } else {
+                spent = max(spent, (uint32_t)__builtin_amdgcn_readfirstlane((int)*(volatile uint32_t*)&s_spent));
+            }
+            while (got < need && spent < (uint32_t)kTraceSegs) {
+                const uint32_t seg = (xcd + spent) % kTraceSegs, size = seg_size(seg), want = need - got;
+                uint32_t base = 0;
+                if (__lane_id() == 0)
+                    base = atomicAdd(reinterpret_cast<uint32_t*>(&a.counters[kSegCounter0 + seg * kSegCounterStride]), want);
+                base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base) + first_fetched(seg);
+                const uint32_t take = base < size ? min(want, size - base) : 0u;
+                if (rank >= got && rank < got + take) {
+                    given = true;
+                    mine = seg * seg_len + base + (rank - got);
+                }
                 got += take;
                 if (base + want >= size) {
-                    seg = (seg + 1) % kTraceSegs;
                     ++spent;
+                    if (__lane_id() == 0) atomicMax(&s_spent, spent);
                 }
             }
-            if (spent >= (unsigned)kTraceSegs) exhausted = true;
+            if (spent >= (uint32_t)kTraceSegs) exhausted = true;
             if (!active) {
-                const int64_t my = (int64_t)mine;
-                if (mine < (unsigned long long)n) {
-                    ray_id = (uint32_t)my;
-                    any_ray = ANY || (DUAL && my >= n1);
-                    const float4* rp = reinterpret_cast<const float4*>(DUAL && my >= n1 ? a.rays2 + (my - n1) : a.rays + my);
+                if (given) {
+                    ray_id = mine;
+                    any_ray = ANY || (DUAL && mine >= n1);
+                    const float4* rp = reinterpret_cast<const float4*>(
+                        DUAL && mine >= n1 ? a.rays2 + (mine - n1) : a.rays + mine);
                     float4 o4 = rp[0], d4 = rp[1];
                     ray_setup(r, mk(o4.x, o4.y, o4.z), mk(d4.x, d4.y, d4.z), d4.w);
                     cur = a.rooted ? __float_as_uint(o4.w) : 0u;
@@ -499,11 +551,17 @@ __global__ void __launch_bounds__(kBlock, (kTraceWaves<KIND, STATS>)) k_trace4(T
         if (active && cur == kNoNode && stash == kNoNode) finish();
     }
 
-    // the last wave of the grid resets the fetch counters for the next launch
-    if (__lane_id() == 0) {
-        unsigned long long prev = atomicAdd(&a.counters[1], 1ull);
-        if (prev == part - 1ull) {
-            for (int k = 0; k < kTraceSegs; ++k) atomicExch(&a.counters[kSegCounter0 + k * kSegCounterStride], 0ull);
+    // the last wave of a long launch resets the counters for the next one
+    // (counted per XCD first: 7,168 waves adding to one address queue for some
+    // 40 us at the end of a launch)
+    if (!shared_out && __lane_id() == 0) {
+        const unsigned long long waves = first_fetched(xcd) / 64u;
+        if (atomicAdd(&a.counters[kSegCounter0 + xcd * kSegCounterStride + kSegDone], 1ull) == waves - 1ull &&
+            atomicAdd(&a.counters[1], 1ull) == kTraceSegs - 1ull) {
+            for (int k = 0; k < kTraceSegs; ++k) {
+                atomicExch(&a.counters[kSegCounter0 + k * kSegCounterStride], 0ull);
+                atomicExch(&a.counters[kSegCounter0 + k * kSegCounterStride + kSegDone], 0ull);
+            }
             atomicExch(&a.counters[1], 0ull);
         }
     }
@@ -555,6 +613,13 @@ int noalloc_setup(int device, hipStream_t stream) {
     return ILM_OK;
 }
 
+// Workgroups that n rays can use: a wave per ray while those are few enough
+// to be dealt out so, a wave per 64 rays of more.
+static int64_t useful_blocks(int64_t n, int cu_count) {
+    const int64_t waves = std::max(std::min<int64_t>(n, (int64_t)cu_count * kShortWaves), (n + 63) / 64);
+    return (waves + kBlock / 64 - 1) / (kBlock / 64);
+}
+
 template <bool ANY, bool STATS, bool DUAL = false>
 static int launch_trace(ilm_mesh* m, const ilm_ray* rays, int64_t n, ilm_hit* hits, uint8_t* occ, int32_t* stats,
                         void* stream, const unsigned long long* n_dev = nullptr, bool rooted = false,
@@ -585,9 +650,8 @@ static int launch_trace(ilm_mesh* m, const ilm_ray* rays, int64_t n, ilm_hit* hi
     int per_cu = 0;
     ILM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, 0));
     per_cu = std::max(per_cu, 1);
-    int64_t blocks = (int64_t)per_cu * ctx->cu_count;
-    blocks = std::min<int64_t>(blocks, (total + kBlock - 1) / kBlock);
-    blocks = std::max<int64_t>(blocks, 1);
+    const int64_t blocks_full = std::max<int64_t>((total + kBlock - 1) / kBlock, 1);  // with a ray in every lane
+    int64_t blocks = std::min<int64_t>((int64_t)per_cu * ctx->cu_count, useful_blocks(total, ctx->cu_count));
     TraceArgs a;
     a.nodes = reinterpret_cast<const float4*>(m->d_nodes);
     a.tris = reinterpret_cast<const float4*>(m->d_tris);
@@ -610,7 +674,7 @@ static int launch_trace(ilm_mesh* m, const ilm_ray* rays, int64_t n, ilm_hit* hi
         a.spill_depth = std::max(1, m->info.stack_need + 1 - keep);
         const int64_t per_block = (int64_t)a.spill_depth * kBlock * (int64_t)sizeof(uint32_t);
         const int64_t fit = (int64_t)(kScratchBytes - kScratchCounterBytes) / per_block;
-        if (fit < std::min<int64_t>(blocks, ctx->cu_count))
+        if (fit < std::min({blocks, blocks_full, (int64_t)ctx->cu_count}))
             return fail(ILM_ERR_INVALID, "tree too deep for the fixed scratch (stack need " +
                                              std::to_string(m->info.stack_need) + ", 64 MiB scratch)");
         blocks = std::min<int64_t>(blocks, fit);
@@ -625,6 +689,7 @@ static int launch_trace(ilm_mesh* m, const ilm_ray* rays, int64_t n, ilm_hit* hi
         a.counters = ctx->counters;
     }
     a.total_waves = (uint32_t)(blocks * (kBlock / 64));
+    a.short_waves = std::min<uint32_t>(a.total_waves, (uint32_t)ctx->cu_count * kShortWaves);
     a.rays2 = DUAL ? q2->rays : nullptr;
     a.n2 = DUAL ? q2->capacity : 0;
     a.n2_dev = DUAL ? q2->n_dev : nullptr;
@@ -658,8 +723,7 @@ int launch_trace_inst(ilm_ctx* ctx, const void* tlas, const void* blas, const fl
     int per_cu = 0;
     ILM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, 0));
     per_cu = std::max(per_cu, 1);
-    int64_t blocks = std::min<int64_t>((int64_t)per_cu * ctx->cu_count, (n + kBlock - 1) / kBlock);
-    blocks = std::max<int64_t>(blocks, 1);
+    const int64_t blocks = std::min<int64_t>((int64_t)per_cu * ctx->cu_count, useful_blocks(n, ctx->cu_count));
     TraceArgs a{};
     a.nodes = reinterpret_cast<const float4*>(blas);
     a.tris = reinterpret_cast<const float4*>(tris);
@@ -675,6 +739,7 @@ int launch_trace_inst(ilm_ctx* ctx, const void* tlas, const void* blas, const fl
     a.spill = ctx->spill;
     a.counters = ctx->counters;
     a.total_waves = (uint32_t)(blocks * (kBlock / 64));
+    a.short_waves = std::min<uint32_t>(a.total_waves, (uint32_t)ctx->cu_count * kShortWaves);
     a.tlas = reinterpret_cast<const float4*>(tlas);
     a.inst = inst;
     a.inst_out = inst_out;

@@ -345,6 +345,51 @@ def _classify_disagreements(orc, om, pos, idx, rays, ph, th, pc, tc):
     return ns.mean(), (ns.sum() + out["bvhmesh"]) / n, out, others, zero_dir
 
 
+@pytest.mark.parametrize("any_hit", [False, True])
+def test_ray_counts_around_the_shares_of_a_launch(any_hit, gpu_ctx, ilm):
+    """A launch deals its rays out to the waves (1 to 64 each) and fetches the
+    rest of a long one by counters: at counts around each of these lines every
+    output equals, bit for bit, that of the same ray in short launches, and
+    nothing past the last is written. The shares depend on the CU count; the
+    grid has at most 8 workgroups of 256 per CU."""
+    pos, idx = meshgen.icosphere(3)
+    m = ilm.Mesh(gpu_ctx, pos, idx)
+    cus = gpu_ctx.cu_count
+    most = 3 * cus * 8 * 256 + 77
+    rng = np.random.default_rng(3)
+    few = meshgen.rays_toward(4000, pos, seed=4)
+    rays = few[rng.integers(len(few), size=most)]
+    rb, fb = ilm.rays_to_device(gpu_ctx, rays), ilm.rays_to_device(gpu_ctx, few)
+    size = 1 if any_hit else 16
+    out, ref = gpu_ctx.buffer((most + 64) * size), gpu_ctx.buffer(len(few) * size)
+    kind = np.dtype(np.uint8) if any_hit else ilm.HIT_DTYPE
+    lines = [8 * cus, 64 * 8 * cus] + [64 * 4 * k * cus for k in range(4, 9)] + [2 * 64 * 4 * 7 * cus]
+    counts = sorted({n + d for n in lines for d in (-1, 0, 1, 13)} | {most})
+    for width, fmt in ((4, 0), (4, 1), (2, 0)):
+        m.build(node_format=fmt, width=width)
+        trace = m.trace_any if any_hit else m.trace_closest
+        for at in range(0, len(few), 500):      # short launches of 500
+            part, o = gpu_ctx.to_device(few[at:at + 500]), gpu_ctx.buffer(500 * size)
+            trace(part, 500, o)
+            gpu_ctx.sync()
+            ref.upload(o.download(np.uint8, 500 * size), at * size)
+            part.free()
+            o.free()
+        want = ref.download(kind, len(few))
+        rng = np.random.default_rng(3)
+        want = want[rng.integers(len(few), size=most)]
+        for n in counts:
+            out.upload(np.full((most + 64) * size, 0xA5, np.uint8))
+            trace(rb, n, out)
+            gpu_ctx.sync()
+            got = out.download(np.uint8, (n + 64) * size)
+            assert np.array_equal(got[:n * size], want[:n].view(np.uint8)), (width, fmt, n)
+            assert (got[n * size:] == 0xA5).all(), (width, fmt, n)
+    for x in (rb, fb, out, ref):
+        x.free()
+    m.close()
+
+
 @pytest.mark.parametrize("ntri", [5, 8, 255, 256, 257, 511, 513, 65535, 65537, 140001])
 def test_lbvh_boxes_are_tight(ntri, gpu_ctx, ilm):
     """Every child's box is exactly the union of its triangles' boxes (unions
