@@ -487,9 +487,13 @@ __global__ void __launch_bounds__(kBlock, (kTraceWaves<KIND, STATS>)) k_trace4(T
             }
             uint32_t cw[W];
 #pragma unroll
-            for (int k = 0; k < W; ++k)  // stage byte offset | slot * 4 (the offset's low bits are clear)
-                cw[k] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(lds) +
-                                                           (stage_off | (key[k] & ((W - 1) << 2))));
+            for (int k = 0; k < W; ++k) {
+                // stage byte offset | slot * 4 (the offset's low bits are
+                // clear): one instruction, which the compiler splits in two
+                uint32_t at;
+                asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(at) : "v"(key[k]), "n"((W - 1) << 2), "v"(stage_off));
+                cw[k] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(lds) + at);
+            }
             // farthest first; a missed child (sorted last, or anywhere in an
             // any-hit launch) is written at the top and left there for the
             // next write to overwrite

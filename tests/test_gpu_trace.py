@@ -345,6 +345,35 @@ def _classify_disagreements(orc, om, pos, idx, rays, ph, th, pc, tc):
     return ns.mean(), (ns.sum() + out["bvhmesh"]) / n, out, others, zero_dir
 
 
+@pytest.mark.parametrize("power", [-51, -40, 0, 40, 60])
+def test_hits_do_not_depend_on_a_power_of_two_scale(power, gpu_ctx, ilm):
+    """Geometry and rays scaled by a power of two: every product and quotient
+    of the ray set-up and the triangle test scales exactly, so t, u, v and the
+    triangle are the same bit for bit, whichever division (the plain one, or
+    the general one for determinants outside [1e-30, 1e30]) is taken."""
+    pos, idx = meshgen.icosphere(3)
+    rays = meshgen.rays_toward(6000, pos, seed=6)
+    d = np.abs(rays[:, 4:7])
+    rays = rays[d.min(axis=1) > 0.01 * d.max(axis=1)]   # no component near the 1e-18 that stands for 0
+    hits = []
+    for e in (0, power):
+        k = np.float32(2.0 ** e)
+        m = ilm.Mesh(gpu_ctx, pos * k, idx)
+        m.build()
+        scaled = rays.copy()
+        scaled[:, 0:3] *= k
+        scaled[:, 4:7] *= k
+        rb, hb = ilm.rays_to_device(gpu_ctx, scaled), gpu_ctx.buffer(len(rays) * 16)
+        m.trace_closest(rb, len(rays), hb)
+        gpu_ctx.sync()
+        hits.append(hb.download(ilm.HIT_DTYPE, len(rays)))
+        rb.free()
+        hb.free()
+        m.close()
+    assert (hits[0]["prim"] >= 0).mean() > 0.3
+    assert np.array_equal(hits[0].view(np.uint32), hits[1].view(np.uint32))
+
+
 @pytest.mark.parametrize("any_hit", [False, True])
 def test_ray_counts_around_the_shares_of_a_launch(any_hit, gpu_ctx, ilm):
     """A launch deals its rays out to the waves (1 to 64 each) and fetches the
