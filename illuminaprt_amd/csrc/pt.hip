@@ -29,6 +29,13 @@ constexpr int kPtBlock = 256;
 // share of the queue) measured fastest; 2 and 4 rounds, and 8 workgroups per
 // CU whatever fits, were slower.
 constexpr int kShadeRounds = 1;
+// Idle lanes by which a bounce's launches wait longer for a refill than the
+// context's threshold: they mix closest hits with shadow segments, which end
+// early and together. Thresholds 20 / 24 / 28 / 32 / 40: 1080p frames 6.09 /
+// 6.09 / 6.06 / 6.09 / 6.13 ms, 256x256 room 1.31 / 1.28 / 1.25 / 1.25 / 1.25,
+// eight rooms 8.14 / 8.00 / 7.93 / 7.90 / 7.89 (closest hits alone are
+// fastest at 16, which the context's default of 24 is near).
+constexpr int kBounceRefill = 4;
 constexpr int kCounts = 16;
 constexpr int kAccumSlots = 4;  // shadow slots per vertex summed from one batch of loads  // the integrator's device counters (PtArgs::counts), cleared per frame
 
@@ -1086,6 +1093,7 @@ int render_views(ilm_scene* s, ilm_nrc* nrc, const std::vector<ilm::View>& views
     a.rr_rule = mode ? mode->rr_rule : 0;
     a.emit0 = mode ? (mode->emit0 ? 1 : 0) : 1;
     hipStream_t st = ctx->stream;
+    const int bounce_refill = std::min(ctx->trace_refill + ilm::kBounceRefill, 64);
     int ev0 = 0, ev1 = 0;
     if (cache && !s->side) {
         // the side stream of cache frames, created before the frame's timing starts
@@ -1123,8 +1131,8 @@ int render_views(ilm_scene* s, ilm_nrc* nrc, const std::vector<ilm::View>& views
             hipLaunchKernelGGL(ilm::k_generate, dim3((unsigned)((a.npaths + 255) / 256)), dim3(256), 0, st, a);
             int cur = 0;
             // camera rays are coherent: their waves refill only when 56 lanes
-            // are idle (measured fastest for primary rays); later launches use
-            // the context's threshold
+            // are idle (measured fastest for primary rays); later launches go
+            // by the context's threshold
             int r2 = ilm::trace_queue(s->mesh, a.rays[0], a.counts + 0, cap, a.hits, nullptr, st, true, 56);
             if (r2) return r2;
             bool forked = false;  // the cache inference of this batch runs on the side stream
@@ -1154,9 +1162,10 @@ int render_views(ilm_scene* s, ilm_nrc* nrc, const std::vector<ilm::View>& views
                 const bool next = b + 1 < max_bounces;
                 if (s->nlights > 0 && next)
                     r2 = ilm::trace_queue_dual(s->mesh, a.rays[cur ^ 1], a.counts + (cur ^ 1), cap, a.hits, a.srays,
-                                               a.counts + 2, cap * max_vl, a.socc, st, true);
+                                               a.counts + 2, cap * max_vl, a.socc, st, true, bounce_refill);
                 else if (s->nlights > 0)
-                    r2 = ilm::trace_queue(s->mesh, a.srays, a.counts + 2, cap * max_vl, nullptr, a.socc, st, true);
+                    r2 = ilm::trace_queue(s->mesh, a.srays, a.counts + 2, cap * max_vl, nullptr, a.socc, st, true,
+                                          bounce_refill);
                 else if (next)
                     r2 = ilm::trace_queue(s->mesh, a.rays[cur ^ 1], a.counts + (cur ^ 1), cap, a.hits, nullptr, st,
                                           true);
