@@ -313,10 +313,10 @@ __global__ void __launch_bounds__(64 * kInferWaves, 6) k_infer(InferArgs a) {
 //
 // Before, one kernel stored all activations and gradients for a second one
 // (98 MB written and read back per 65,536 samples). Steps of 65,536 samples,
-// Adam included, 61.4 -> 36.5 us; 4,096 samples 29.4 -> 17.1 us; 262,144 312
-// -> 81 us. What bounds it: 7.4 us per 128 samples and CU, a chain of layers
+// Adam included, 61.4 -> 35.1 us; 4,096 samples 29.4 -> 16.4 us; 262,144 312
+// -> 74 us. What bounds it: 6.5 us per 128 samples and CU, a chain of layers
 // with one workgroup per CU (160 KB of LDS) whose LDS serves the weights'
-// fragments, the staging and the reductions (~11,000 of the 18,000 cycles);
+// fragments, the staging and the reductions (~11,000 of the 15,600 cycles);
 // and the workgroups' sums, 94 KB each, 10 us to write for 256 of them.
 constexpr int kTrainWaves = 8;
 constexpr int kTrainSamples = 16 * kTrainWaves;
@@ -379,9 +379,13 @@ __device__ __forceinline__ void store_tiles(const f32x4 (&acc)[N], float* part, 
 
 // ReLU's derivative of 16 outputs kept in one register: bits k and 16 + k tell
 // whether the two halves of pair k (bf16, never below 0) are above 0.
+// One instruction (a 16-bit minimum with 1); written as a minimum, the
+// compiler makes a compare and a select of each half (7.4 us per 128 samples
+// and CU instead of 6.5).
 __device__ __forceinline__ unsigned positive_bits(unsigned pair) {
-    const u16x2 one = __builtin_elementwise_min(__builtin_bit_cast(u16x2, pair), (u16x2)(unsigned short)1);
-    return __builtin_bit_cast(unsigned, one);
+    unsigned one;
+    asm("v_pk_min_u16 %0, %1, 1 op_sel_hi:[1,0]" : "=v"(one) : "v"(pair));
+    return one;
 }
 __device__ __forceinline__ unsigned halves_mask(unsigned bits) {  // 0x0000 or 0xFFFF per half from its lowest bit
     return __builtin_bit_cast(unsigned, (u16x2)(unsigned short)0 - __builtin_bit_cast(u16x2, bits));
