@@ -129,6 +129,7 @@ SIGNATURES = {
     "ilm_device_count": (C.c_int, [C.POINTER(C.c_int)]),
     "ilm_device_info": (C.c_int, [_vp, C.c_char_p, C.c_int, C.POINTER(C.c_int)]),
     "ilm_device_memory": (C.c_int, [_vp, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]),
+    "ilm_ctx_fail_allocations": (C.c_int, [_vp, _i64, _i64]),
     "ilm_ctx_set_trace_refill": (C.c_int, [_vp, C.c_int]),
     "ilm_alloc": (C.c_int, [_vp, _sz, C.POINTER(_vp)]),
     "ilm_free": (C.c_int, [_vp, _vp]),
@@ -322,6 +323,10 @@ class Context:
 
     def set_trace_refill(self, idle_lanes: int):
         check(load().ilm_ctx_set_trace_refill(self.h, idle_lanes))
+
+    def fail_allocations(self, skip: int = 0, count: int = 0):
+        """For tests: after `skip` device allocations, refuse the next `count`."""
+        check(load().ilm_ctx_fail_allocations(self.h, skip, count))
 
     def memory(self) -> tuple[int, int]:
         """(free, total) bytes of device memory."""

@@ -28,6 +28,25 @@ hipStream_t pick_stream(ilm_ctx* ctx, void* stream) {
     return stream ? (hipStream_t)stream : ctx->stream;
 }
 
+hipError_t device_malloc(ilm_ctx* ctx, void** p, size_t bytes) {
+    *p = nullptr;
+    {
+        std::lock_guard<std::mutex> g(ctx->mu);
+        if (ctx->alloc_skip > 0) {
+            --ctx->alloc_skip;
+        } else if (ctx->alloc_fail > 0) {
+            --ctx->alloc_fail;
+            return hipErrorOutOfMemory;
+        }
+    }
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
 int ensure_spill(ilm_ctx* ctx, size_t words) {
     if (ctx->spill_words >= words) return ILM_OK;
     if (ctx->spill) {
@@ -147,17 +166,16 @@ int ilm_alloc(ilm_ctx* ctx, size_t bytes, void** dev) {
     if (bytes == 0) bytes = 16;
     ILM_HIP(hipSetDevice(ctx->device));
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
+    hipError_t e = ilm::device_malloc(ctx, &p, bytes);
     if (e == hipErrorOutOfMemory) {
         // the kept build workspace makes room, unless a build uses it
         ilm::BuildWorkspace held(ctx, true);
         if (held.mine && ctx->build_ws) {
-            (void)hipGetLastError();
             ILM_HIP(hipStreamSynchronize(ctx->stream));
             ILM_HIP(hipFree(ctx->build_ws));
             ctx->build_ws = nullptr;
             ctx->build_bytes = 0;
-            e = hipMalloc(&p, bytes);
+            e = ilm::device_malloc(ctx, &p, bytes);
         }
     }
     if (e == hipErrorOutOfMemory) return fail(ILM_ERR_NOMEM, "device allocation of " + std::to_string(bytes) + " bytes");
@@ -165,6 +183,14 @@ int ilm_alloc(ilm_ctx* ctx, size_t bytes, void** dev) {
     std::lock_guard<std::mutex> g(ctx->mu);
     ctx->allocs.insert(p);
     *dev = p;
+    return ILM_OK;
+}
+
+int ilm_ctx_fail_allocations(ilm_ctx* ctx, int64_t skip, int64_t count) {
+    if (!ctx || skip < 0 || count < 0) return fail(ILM_ERR_INVALID, "bad arguments");
+    std::lock_guard<std::mutex> g(ctx->mu);
+    ctx->alloc_skip = count > 0 ? skip : 0;
+    ctx->alloc_fail = count;
     return ILM_OK;
 }
 

@@ -398,6 +398,7 @@ struct ilm_ic {
     float4* d_jobs = nullptr;  // per node with masks: its job, then its bounds (k_ic_masks)
     size_t cap_masks = 0, cap_jobs = 0;
     int grid = 1;
+    bool on_device = false;  // the device copies are whole (an upload may fail for lack of memory)
     uint32_t passes = 0;
     unsigned long long* d_count = nullptr;
     // frame buffers, grown on demand and kept across frames
@@ -485,8 +486,12 @@ float record_reach2(const ilm_ic* ic, const ilm_ic::Rec& r) {
     return reach >= 0.f ? reach * reach * 1.0001f : INFINITY;
 }
 
-// Flattened octree and records to the device, and the masks of its long lists.
+// Flattened octree and records to the device, and the masks of its long
+// lists. Without memory for the masks the lists are walked whole: the nodes
+// say which of them have masks, so they are copied only once the masks' room
+// is there.
 int upload(ilm_ic* ic) {
+    ic->on_device = false;
     std::vector<float> nodes(12 * ic->nodes.size());
     std::vector<int32_t> refs, jobs;
     std::vector<float> bounds;
@@ -494,9 +499,9 @@ int upload(ilm_ic* ic) {
     int32_t longest = 0;
     for (const ilm_ic::Node& n : ic->nodes)
         if (n.recs.size() > (size_t)ilm::kMaskMin) words += ((int64_t)n.recs.size() + 31) / 32;
-    ic->grid = ilm::kMaskGrid;
-    while (ic->grid > 1 && words * ic->grid * ic->grid * ic->grid * 4 > ilm::kMaskBytes) ic->grid /= 2;
-    const int64_t cells = (int64_t)ic->grid * ic->grid * ic->grid;
+    int64_t grid = ilm::kMaskGrid;
+    while (grid > 1 && words * grid * grid * grid * 4 > ilm::kMaskBytes) grid /= 2;
+    const int64_t cells = grid * grid * grid;
     const bool masked = words * cells < INT32_MAX;
     words = 0;
     for (size_t i = 0; i < ic->nodes.size(); ++i) {
@@ -529,22 +534,38 @@ int upload(ilm_ic* ic) {
     int rc = grow(ic->ctx, (void**)&ic->d_nodes, ic->cap_nodes, nodes.size() * 4);
     if (!rc) rc = grow(ic->ctx, (void**)&ic->d_refs, ic->cap_refs, refs.size() * 4);
     if (!rc) rc = grow(ic->ctx, (void**)&ic->d_recs, ic->cap_recs, recs.size() * 4);
+    if (rc) return rc;
+    size_t njobs = jobs.size() / 4;
+    if (njobs > 0) {
+        rc = grow(ic->ctx, (void**)&ic->d_masks, ic->cap_masks, (size_t)words * 4);
+        if (!rc) rc = grow(ic->ctx, (void**)&ic->d_jobs, ic->cap_jobs, njobs * 48);
+        if (rc == ILM_ERR_NOMEM) {
+            njobs = 0;
+            for (size_t i = 0; i < ic->nodes.size(); ++i) nodes[12 * i + 10] = 0.f;  // words per cell
+            if (ic->d_masks) ilm_free(ic->ctx, ic->d_masks);
+            ic->d_masks = nullptr;
+            ic->cap_masks = 0;
+            rc = ILM_OK;
+        }
+    }
     if (!rc) rc = ilm_upload(ic->ctx, ic->d_nodes, nodes.data(), nodes.size() * 4);
     if (!rc) rc = ilm_upload(ic->ctx, ic->d_refs, refs.data(), refs.size() * 4);
     if (!rc) rc = ilm_upload(ic->ctx, ic->d_recs, recs.data(), recs.size() * 4);
-    const size_t njobs = jobs.size() / 4;
-    if (rc || njobs == 0) return rc;
-    rc = grow(ic->ctx, (void**)&ic->d_masks, ic->cap_masks, (size_t)words * 4);
-    if (!rc) rc = grow(ic->ctx, (void**)&ic->d_jobs, ic->cap_jobs, njobs * 48);
-    if (!rc) rc = ilm_upload(ic->ctx, ic->d_jobs, jobs.data(), njobs * 16);
-    if (!rc) rc = ilm_upload(ic->ctx, ic->d_jobs + njobs, bounds.data(), njobs * 32);
+    if (!rc && njobs > 0) {
+        rc = ilm_upload(ic->ctx, ic->d_jobs, jobs.data(), njobs * 16);
+        if (!rc) rc = ilm_upload(ic->ctx, ic->d_jobs + njobs, bounds.data(), njobs * 32);
+        if (rc) return rc;
+        hipLaunchKernelGGL(ilm::k_ic_masks,
+                           dim3((unsigned)njobs, (unsigned)((cells + 63) / 64), (unsigned)std::min(longest, 1024)),
+                           dim3(64), 0, ic->ctx->stream, reinterpret_cast<const int4*>(ic->d_jobs), ic->d_jobs + njobs,
+                           ic->d_refs, ic->d_recs, (int)grid, ic->d_masks);
+        ILM_HIP(hipGetLastError());
+        // lookups may follow on any stream, as after the copies above
+        ILM_HIP(hipStreamSynchronize(ic->ctx->stream));
+    }
     if (rc) return rc;
-    hipLaunchKernelGGL(ilm::k_ic_masks, dim3((unsigned)njobs, (unsigned)((cells + 63) / 64), (unsigned)std::min(longest, 1024)),
-                       dim3(64), 0, ic->ctx->stream, reinterpret_cast<const int4*>(ic->d_jobs), ic->d_jobs + njobs, ic->d_refs,
-                       ic->d_recs, ic->grid, ic->d_masks);
-    ILM_HIP(hipGetLastError());
-    // lookups may follow on any stream, as after the copies above
-    ILM_HIP(hipStreamSynchronize(ic->ctx->stream));
+    ic->grid = (int)grid;
+    ic->on_device = true;
     return ILM_OK;
 }
 
@@ -715,6 +736,10 @@ int ilm_ic_node_records(ilm_ic* ic, int64_t node, int32_t* count, int32_t* child
 int ilm_ic_lookup(ilm_ic* ic, const float* points, int64_t n, float* out, void* stream) {
     if (!ic || n < 0 || (n > 0 && (!points || !out))) return fail(ILM_ERR_INVALID, "bad arguments");
     if (n == 0) return ILM_OK;
+    if (!ic->on_device) {
+        const int rc = upload(ic);
+        if (rc) return rc;
+    }
     hipStream_t st = stream ? (hipStream_t)stream : ic->ctx->stream;
     hipLaunchKernelGGL(ilm::k_ic_lookup_points, dim3(ilm::grid_of(n)), dim3(256), 0, st, args_of(ic), points, n, out);
     ILM_HIP(hipGetLastError());
@@ -748,6 +773,7 @@ int ilm_ic_render(ilm_ic* ic, const ilm_render_params* prm, double* accum, ilm_i
     if (!rc) rc = grow(ic->miss, (size_t)nsamp);
     if (!rc) rc = grow(ic->sel, (size_t)nsamp * 4);
     if (!rc) rc = grow(ic->nsel, 8);
+    if (!rc && !ic->on_device) rc = upload(ic);
     if (rc) return rc;
     float* gbuf = (float*)ic->gbuf.p;
     int32_t* own = (int32_t*)ic->own.p;

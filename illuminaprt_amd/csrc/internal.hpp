@@ -61,6 +61,9 @@ struct ilm_ctx {
     size_t build_bytes = 0;
     std::atomic<bool> build_held{false};
     int trace_refill = 24;  // idle lanes of a wave that trigger its ray refill
+    // device allocations still to succeed, then to be refused
+    // (ilm_ctx_fail_allocations); under mu
+    int64_t alloc_skip = 0, alloc_fail = 0;
     std::mutex mu;
 };
 
@@ -82,6 +85,9 @@ struct ilm_mesh {
 };
 
 namespace ilm {
+// hipMalloc for the context; leaves no error behind for a later
+// hipGetLastError when the device is full.
+hipError_t device_malloc(ilm_ctx* ctx, void** p, size_t bytes);
 // Ensures ctx->spill holds at least `words` 32-bit words.
 int ensure_spill(ilm_ctx* ctx, size_t words);
 // Holds ctx->build_ws for a scope, if it is wanted and no other thread does.

@@ -84,6 +84,11 @@ int ilm_device_info(ilm_ctx* ctx, char* name, int name_len, int* cu_count);
  * used to report a workload's HBM footprint. */
 int ilm_device_memory(ilm_ctx* ctx, uint64_t* free_bytes, uint64_t* total_bytes);
 
+/* For tests of error paths: of the context's device allocations that follow,
+ * `skip` go ahead, the next `count` are refused as on a full device
+ * (ILM_ERR_NOMEM), and later ones go ahead. count 0 ends it. */
+int ilm_ctx_fail_allocations(ilm_ctx* ctx, int64_t skip, int64_t count);
+
 /* Device buffers owned by the context (freed by ilm_ctx_destroy). */
 int ilm_alloc(ilm_ctx* ctx, size_t bytes, void** dev);
 int ilm_free(ilm_ctx* ctx, void* dev);

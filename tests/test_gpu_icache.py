@@ -248,3 +248,52 @@ def test_lookups_at_list_lengths_around_the_masks(gpu_ctx, ilm, variant, count):
         ic.close()
     sc.close()
     m.close()
+
+
+@pytest.mark.parametrize("refused", range(6))
+def test_lookups_after_an_allocation_was_refused(gpu_ctx, ilm, refused):
+    """An insertion whose n-th device allocation (nodes, references, records,
+    masks, their jobs; the sixth does not happen) is refused. Without masks
+    the lists are walked whole, to the same sums bit for bit; without the
+    others the insertion fails, lookups fail while memory is short, and the
+    next one with memory sees every record."""
+    m, sc, pos = _room(ilm, gpu_ctx)
+    rng = np.random.default_rng(4)
+
+    def records(n):
+        N = np.array([0, 1, 0]) + 0.2 * rng.normal(size=(n, 3))
+        N /= np.linalg.norm(N, axis=1, keepdims=True)
+        return np.concatenate([rng.random((n, 3)), N, rng.random((n, 3)), 0.05 + 0.2 * rng.random((n, 1))],
+                              1).astype(np.float32)
+    first, second = records(50), records(4000)
+    Q = np.concatenate([rng.random((2000, 3)), np.tile([0, 1.0, 0], (2000, 1))], 1).astype(np.float32)
+    caches = [ilm.IrradianceCache(sc, cache_depth=4, error_threshold=0.3, ambient_resolution=0.01,
+                                  ambient_multiplier=10.0) for _ in range(2)]
+    for ic in caches:
+        ic.insert(first)
+    whole, short = caches
+    whole.insert(second)
+    want = whole.lookup(Q)
+    assert (want[:, 3] > 0).mean() > 0.3
+    points, out = gpu_ctx.to_device(Q), gpu_ctx.buffer(len(Q) * 16)
+    lookup = lambda: ilm.load().ilm_ic_lookup(short.h, points.ptr, len(Q), out.ptr, None)
+    try:
+        if refused < 3:
+            gpu_ctx.fail_allocations(refused, 1000)
+            with pytest.raises(ilm.IlmError):
+                short.insert(second)
+            assert lookup() == -3  # ILM_ERR_NOMEM
+            gpu_ctx.fail_allocations()
+        else:
+            gpu_ctx.fail_allocations(refused, 2)  # a context tries again after freeing what it keeps
+            short.insert(second)
+            gpu_ctx.fail_allocations()
+        assert np.array_equal(short.lookup(Q).view(np.uint32), want.view(np.uint32))
+        more = records(3)
+        for ic in caches:
+            ic.insert(more)
+        assert np.array_equal(short.lookup(Q).view(np.uint32), whole.lookup(Q).view(np.uint32))
+    finally:
+        gpu_ctx.fail_allocations()
+    for x in (points, out, *caches, sc, m):
+        (x.free if hasattr(x, "free") else x.close)()
