@@ -85,18 +85,20 @@ __device__ __forceinline__ int cell_of(float x, float lo, float scale, int grid)
 // sqrt(x), a / b and 1 / x from the hardware's approximations (1 ulp) and a
 // step that adds the remainder's correction, which leaves them rounded to
 // nearest but for rare ties: a quarter of the instructions of the compiler's
-// forms, which also scale arguments near the ends of the range. Here
-// distances, radii and weights stay far from those: a squared distance of
-// at most 1e-37 is 0 beside the 1 it is added to, radii of 0 have no weight
-// however they divide, and x = 0 gives infinity.
+// forms, which also scale arguments near the ends of the range. At those ends:
+// the root of 0 and infinity is exact, that of a squared distance below the
+// smallest normal float (points 1e-19 apart) is about 0; v_div_fixup_f32
+// gives the quotient its infinities, zeros and NaN (a record's radius is
+// infinite where no gather ray hit and no bound was asked for, 0 in a scene
+// without extent); and 1 / 0 is infinite.
 __device__ __forceinline__ float root_of(float x) {
     const float r = __builtin_amdgcn_rsqf(x), s = x * r;
     const float t = fmaf(fmaf(-s, s, x), 0.5f * r, s);
-    return x > 1e-37f ? t : 0.f * x;
+    return __builtin_amdgcn_classf(x, 0x100) ? t : x;  // 0x100: positive and normal
 }
 __device__ __forceinline__ float ratio_of(float a, float b) {
     const float r = __builtin_amdgcn_rcpf(b), q = a * r;
-    return fmaf(fmaf(-q, b, a), r, q);
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, b, a), r, q), b, a);
 }
 __device__ __forceinline__ float inverse_of(float x) {
     const float r = __builtin_amdgcn_rcpf(x), t = fmaf(fmaf(-x, r, 1.f), r, r);

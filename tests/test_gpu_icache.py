@@ -297,3 +297,45 @@ def test_lookups_after_an_allocation_was_refused(gpu_ctx, ilm, refused):
         gpu_ctx.fail_allocations()
     for x in (points, out, *caches, sc, m):
         (x.free if hasattr(x, "free") else x.close)()
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("count", [1, 32, 33, 70])
+def test_records_of_infinite_radius_keep_their_weight(gpu_ctx, ilm, variant, count):
+    """An unbounded ambient_multiplier leaves a record whose gather rays all
+    miss its infinite radius. Its distance then counts nothing and its weight
+    is that of the normals alone, 1 / (1 - cos) - 1 / threshold (Ward) or 1 -
+    9.0124 (1 - cos) / threshold: in 64 bits, off by the rounding of 1 - cos
+    (four roundings of 2^-24) over its square, and of the sum."""
+    m, sc, pos = _room(ilm, gpu_ctx)
+    threshold = 0.5
+    ic = ilm.IrradianceCache(sc, cache_depth=2, error_threshold=threshold, ambient_resolution=0.01,
+                             ambient_multiplier=float("inf"), variant=variant)
+    rng = np.random.default_rng(count)
+    a = 0.15 + 0.2 * rng.random(count)                   # radians off the lookups' normal
+    N = np.stack([np.sin(a), np.cos(a), np.zeros(count)], 1)
+    R = np.concatenate([rng.random((count, 3)), N, rng.random((count, 3)), np.full((count, 1), np.inf)],
+                       1).astype(np.float32)
+    R[::5, 9] = 0.02                                     # and a few that reach no lookup
+    if count == 1:
+        R[0, 9] = np.inf
+    ic.insert(R)
+    far = np.isinf(ic.records()[:, 10])
+    assert far.sum() >= max(1, 0.7 * count)
+    q = 200
+    Q = np.concatenate([np.full((q, 3), 0.98) + 0.01 * rng.random((q, 3)), np.tile([0, 1.0, 0], (q, 1))],
+                       1).astype(np.float32)
+    got = ic.lookup(Q).astype(np.float64)
+    x = 1 - R[far, 4].astype(np.float64)
+    w = 1 / x - 1 / threshold if variant == 0 else 1 - 9.0124 * x / threshold
+    off = 4 * 2.0 ** -24 * ((1 / x ** 2 + 1 / x) if variant == 0 else np.full(len(x), 9.0124 / threshold + 1))
+    w0 = np.maximum(w, 0)
+    den, bound = w0.sum(), off.sum() + count * 2.0 ** -23 * w0.sum()
+    assert den > 100 * bound
+    clear = ~(np.linalg.norm(Q[:, None, :3] - R[None, ~far, :3], axis=2).min(axis=1, initial=9.0) < 0.02)
+    assert clear.sum() > q / 2
+    assert np.abs(got[clear, 3] - den).max() <= bound
+    e = (w0[:, None] * R[far, 6:9]).sum(0) / den
+    assert np.abs(got[clear, :3] - e).max() <= 2 * bound / den + count * 2.0 ** -23
+    for x in (ic, sc, m):
+        x.close()
