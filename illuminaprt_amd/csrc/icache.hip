@@ -53,7 +53,10 @@ namespace {
 constexpr float kPiF = 3.14159265358979323846f;
 // Lists up to kMaskMin records are tested whole: one word of mask would save
 // less than it costs to read. A node with masks has up to kMaskGrid cells per
-// axis, fewer while the masks of all nodes would exceed kMaskBytes.
+// axis, fewer while the masks of all nodes would exceed kMaskBytes. Two 1080p
+// frames of the 1.31M-triangle scene at thresholds 0.3 / 0.5 / 1 (Ward): a
+// grid of 4 20.4 / 20.9 / 30.8 ms, of 8 18.9 / 19.1 / 29.0, of 16 21.4 / 20.0
+// / 28.0; lists from 17 or 65 records on within 1% of these.
 constexpr int kMaskMin = 32, kMaskGrid = 8;
 constexpr int64_t kMaskBytes = int64_t(128) << 20;
 constexpr float kUnitNormal2 = 1.0001f;  // squared length of a lookup normal the masks hold for
@@ -116,16 +119,44 @@ __device__ __forceinline__ float ic_weight(const IcArgs& c, float rc, f3 rn, flo
     return cosv <= 0.f ? 0.f : inverse_of(dist + 1.f - cosv) - c.inv_threshold;
 }
 
+// How a lookup walks the lists (the sums are the same bit for bit): through
+// the masks, a record's position loaded first and the rest only within its
+// reach; through the masks, a record's 48 bytes loaded at once; or whole.
+// A record's reach grows with the threshold, and with it the share of the
+// tests that pass, for which loads one after another only wait longer, and
+// the share of a cell's bits that are set. Frames, whose lanes are
+// neighbouring pixels, go by the masks and the reach at every threshold (two
+// 1080p frames of the 1.31M-triangle scene, Ward, masks / whole lists: 19.2 /
+// 46.8 ms at 0.3, 28.9 / 38.6 at 1, 33.1 / 34.9 at 2). A caller's points may
+// lie anywhere; 1M points at random records of that scene, and the same
+// points sorted by record, in ms:
+//   threshold       0.3          0.75         0.9         1          1.25        1.5
+//   reach        4.1 /  1.1  11.6 / 3.8  14.3 / 5.1  16.6 / 6.2  20.7 / 7.9  22.3 /  8.8
+//   at once      3.7 /  1.2   9.1 / 4.5  11.2 / 5.9  13.1 / 7.2  15.7 / 9.0  17.0 / 10.1
+//   whole       15.4 /  7.9  15.3 / 8.4  15.3 / 8.5  15.3 / 8.6  15.3 / 8.7  15.3 /  8.7
+// (whole lists before there were masks: 15.6 / 8.2 to 9.0). So points go by
+// the reach up to kReachThreshold, by the masks up to kMaskThreshold.
+enum { kWalkReach, kWalkAtOnce, kWalkWhole };
+constexpr float kReachThreshold = 0.9f, kMaskThreshold = 1.2f;
+
 // Adds the share of record r (this lane's own) at (p, n); far: skip it beyond its reach.
+template <int WALK>
 __device__ __forceinline__ void ic_add(const IcArgs& c, int r, bool far, f3 p, f3 n, f3& e, float& den) {
     const float4 pr = c.recs[3 * r];
+    float4 nr, er;
+    if (WALK != kWalkReach) {
+        nr = c.recs[3 * r + 1];
+        er = c.recs[3 * r + 2];
+    }
     const float dx = p.x - pr.x, dy = p.y - pr.y, dz = p.z - pr.z;
     const float d2 = dx * dx + dy * dy + dz * dz;
-    if (far && d2 > pr.w) return;
-    const float4 nr = c.recs[3 * r + 1];
+    if (WALK == kWalkReach) {
+        if (far && d2 > pr.w) return;
+        nr = c.recs[3 * r + 1];
+    }
     const float w = ic_weight(c, nr.w, mk(nr.x, nr.y, nr.z), d2, n);
     if (w > 0.f) {
-        const float4 er = c.recs[3 * r + 2];
+        if (WALK == kWalkReach) er = c.recs[3 * r + 2];
         e = e + w * mk(er.x, er.y, er.z);
         den += w;
     }
@@ -145,11 +176,10 @@ __device__ __forceinline__ void ic_add(const IcArgs& c, int r, bool far, f3 p, f
 // records, its masks leave 415 and 210 of them have weight: 2.07M lookups
 // take 1.5 ms (13.7 ms over the whole lists). Walking the lists that a wave's
 // lanes share with scalar loads was slower (2.6 ms): the lanes then wait for
-// each other's lists and one record at a time. A grid of 4 cells per axis
-// leaves more records, one of 16 takes eight times the masks and their time.
+// each other's lists and one record at a time.
 // ANY: only whether some record has weight there is asked (the sum's sign):
 // the walk ends at the first (2.07M lookups 1.5 -> 0.6 ms).
-template <bool ANY>
+template <bool ANY, int WALK = kWalkReach>
 __device__ float ic_lookup(const IcArgs& c, f3 p, f3 n, f3& e) {
     e = mk(0, 0, 0);
     float den = 0.f;
@@ -161,7 +191,7 @@ __device__ float ic_lookup(const IcArgs& c, f3 p, f3 n, f3& e) {
     for (int level = 0; level < 64; ++level) {
         const float4 lo = c.nodes[3 * node], hi = c.nodes[3 * node + 1], cnt = c.nodes[3 * node + 2];
         const int first = __float_as_int(hi.w), count = __float_as_int(cnt.x);
-        const int words = unit ? __float_as_int(cnt.z) : 0;
+        const int words = unit && WALK != kWalkWhole ? __float_as_int(cnt.z) : 0;
         if (words) {
             const float g = (float)c.grid;
             const int cx = cell_of(p.x, lo.x, g / (hi.x - lo.x), c.grid);
@@ -172,13 +202,13 @@ __device__ float ic_lookup(const IcArgs& c, f3 p, f3 n, f3& e) {
             for (int q = -1;;) {
                 while (left == 0 && ++q < words) left = m[q];
                 if (left == 0) break;
-                ic_add(c, c.refs[first + 32 * q + __ffs((int)left) - 1], true, p, n, e, den);
+                ic_add<WALK>(c, c.refs[first + 32 * q + __ffs((int)left) - 1], true, p, n, e, den);
                 if (ANY && den > 0.f) return den;
                 left &= left - 1u;
             }
         } else {
             for (int k = 0; k < count; ++k) {
-                ic_add(c, c.refs[first + k], unit, p, n, e, den);
+                ic_add<WALK>(c, c.refs[first + k], unit, p, n, e, den);
                 if (ANY && den > 0.f) return den;
             }
         }
@@ -349,12 +379,13 @@ __global__ void k_ic_shade(IcArgs c, const float4* gbuf, const int32_t* own, int
     if (looked) atomicAdd(lookups, (unsigned long long)looked);
 }
 
+template <int WALK>
 __global__ void k_ic_lookup_points(IcArgs c, const float* pts, int64_t n, float* out) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     f3 e;
     const float* q = pts + 6 * i;
-    const float w = ic_lookup<false>(c, mk(q[0], q[1], q[2]), mk(q[3], q[4], q[5]), e);
+    const float w = ic_lookup<false, WALK>(c, mk(q[0], q[1], q[2]), mk(q[3], q[4], q[5]), e);
     out[4 * i] = e.x;
     out[4 * i + 1] = e.y;
     out[4 * i + 2] = e.z;
@@ -550,22 +581,30 @@ int upload(ilm_ic* ic) {
             rc = ILM_OK;
         }
     }
-    if (!rc) rc = ilm_upload(ic->ctx, ic->d_nodes, nodes.data(), nodes.size() * 4);
-    if (!rc) rc = ilm_upload(ic->ctx, ic->d_refs, refs.data(), refs.size() * 4);
-    if (!rc) rc = ilm_upload(ic->ctx, ic->d_recs, recs.data(), recs.size() * 4);
-    if (!rc && njobs > 0) {
-        rc = ilm_upload(ic->ctx, ic->d_jobs, jobs.data(), njobs * 16);
-        if (!rc) rc = ilm_upload(ic->ctx, ic->d_jobs + njobs, bounds.data(), njobs * 32);
-        if (rc) return rc;
-        hipLaunchKernelGGL(ilm::k_ic_masks,
-                           dim3((unsigned)njobs, (unsigned)((cells + 63) / 64), (unsigned)std::min(longest, 1024)),
-                           dim3(64), 0, ic->ctx->stream, reinterpret_cast<const int4*>(ic->d_jobs), ic->d_jobs + njobs,
-                           ic->d_refs, ic->d_recs, (int)grid, ic->d_masks);
-        ILM_HIP(hipGetLastError());
-        // lookups may follow on any stream, as after the copies above
-        ILM_HIP(hipStreamSynchronize(ic->ctx->stream));
-    }
     if (rc) return rc;
+    // copies and masks on the context's stream, one wait for all of them:
+    // lookups may follow on any stream
+    hipStream_t st = ic->ctx->stream;
+    auto put = [&](void* dev, const void* host, size_t bytes) {
+        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
+    };
+    hipError_t err = put(ic->d_nodes, nodes.data(), nodes.size() * 4);
+    if (err == hipSuccess) err = put(ic->d_refs, refs.data(), refs.size() * 4);
+    if (err == hipSuccess) err = put(ic->d_recs, recs.data(), recs.size() * 4);
+    if (err == hipSuccess && njobs > 0) {
+        err = put(ic->d_jobs, jobs.data(), njobs * 16);
+        if (err == hipSuccess) err = put(ic->d_jobs + njobs, bounds.data(), njobs * 32);
+        if (err == hipSuccess) {
+            hipLaunchKernelGGL(ilm::k_ic_masks,
+                               dim3((unsigned)njobs, (unsigned)((cells + 63) / 64), (unsigned)std::min(longest, 1024)),
+                               dim3(64), 0, st, reinterpret_cast<const int4*>(ic->d_jobs), ic->d_jobs + njobs,
+                               ic->d_refs, ic->d_recs, (int)grid, ic->d_masks);
+            err = hipGetLastError();
+        }
+    }
+    const hipError_t waited = hipStreamSynchronize(st);
+    if (err == hipSuccess) err = waited;
+    if (err != hipSuccess) return ilm::fail_hip(err, "irradiance cache upload");
     ic->grid = (int)grid;
     ic->on_device = true;
     return ILM_OK;
@@ -743,7 +782,11 @@ int ilm_ic_lookup(ilm_ic* ic, const float* points, int64_t n, float* out, void* 
         if (rc) return rc;
     }
     hipStream_t st = stream ? (hipStream_t)stream : ic->ctx->stream;
-    hipLaunchKernelGGL(ilm::k_ic_lookup_points, dim3(ilm::grid_of(n)), dim3(256), 0, st, args_of(ic), points, n, out);
+    const float threshold = ic->prm.error_threshold;
+    auto* kernel = threshold <= ilm::kReachThreshold  ? ilm::k_ic_lookup_points<ilm::kWalkReach>
+                   : threshold <= ilm::kMaskThreshold ? ilm::k_ic_lookup_points<ilm::kWalkAtOnce>
+                                                      : ilm::k_ic_lookup_points<ilm::kWalkWhole>;
+    hipLaunchKernelGGL(kernel, dim3(ilm::grid_of(n)), dim3(256), 0, st, args_of(ic), points, n, out);
     ILM_HIP(hipGetLastError());
     return ILM_OK;
 }

@@ -339,3 +339,56 @@ def test_records_of_infinite_radius_keep_their_weight(gpu_ctx, ilm, variant, cou
     assert np.abs(got[clear, :3] - e).max() <= 2 * bound / den + count * 2.0 ** -23
     for x in (ic, sc, m):
         x.close()
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("threshold", [0.9, 0.95, 1.2, 1.25])
+def test_lookups_on_both_sides_of_the_thresholds_of_the_walk(gpu_ctx, ilm, variant, threshold):
+    """Lookups of points walk the lists by the records' reach, by the masks
+    alone or whole, depending on the threshold. Lists of 33 and 150 records
+    (with and without whole words of mask), against the sums in 64 bits: a
+    weight 1 / x - 1 / threshold, x = d / RiClamp + 1 - cos, is off by x's
+    rounding (24 roundings of its terms) over x squared and its own, Tabelion's
+    by 48, and a list's sum by its length times 2^-23."""
+    m, sc, pos = _room(ilm, gpu_ctx)
+    rng = np.random.default_rng(12)
+    inv = float(np.float32(1) / np.float32(threshold))
+    for count in (33, 150):
+        ic = ilm.IrradianceCache(sc, cache_depth=1, error_threshold=threshold, ambient_resolution=0.01,
+                                 ambient_multiplier=10.0, variant=variant)
+        N = np.array([0, 1, 0]) + 0.3 * rng.normal(size=(count, 3))
+        N /= np.linalg.norm(N, axis=1, keepdims=True)
+        R = np.concatenate([rng.random((count, 3)) * 0.4 + 0.05, N, rng.random((count, 3)),
+                            0.02 + 0.1 * rng.random((count, 1))], 1).astype(np.float32)
+        ic.insert(R)
+        lists = [ic.node(k)[1] for k in range(ic.info()["nodes"])]
+        lo, hi = ic.info()["root"][:3], ic.info()["root"][3:]
+        centre = lo + (hi - lo) * np.float32(0.5)
+        Q = np.concatenate([rng.random((400, 3)) * 0.5, np.tile([0, 1.0, 0], (400, 1))], 1).astype(np.float32)
+        got = ic.lookup(Q).astype(np.float64)
+        rc, Rd, Qd = ic.records()[:, 10].astype(np.float64), R.astype(np.float64), Q.astype(np.float64)
+        weighted = 0
+        for i in range(len(Q)):
+            b = Q[i, :3] > centre
+            r = lists[1 + int(b[0]) + 2 * int(b[2]) + 4 * int(b[1])]
+            d = np.linalg.norm(Rd[r, :3] - Qd[i, :3], axis=1) / rc[r]
+            cos = Rd[r, 3:6] @ Qd[i, 3:]
+            if variant == 0:
+                x = d + 1 - cos
+                w = np.where(cos > 0, 1 / x - inv, -1.0)
+                off = 24 * 2.0 ** -24 * np.maximum(d, 1) / x ** 2 + 4 * 2.0 ** -24 * (np.abs(1 / x) + inv)
+            else:
+                w = 1 - inv * np.maximum(d, (1 - cos) * 9.0124)
+                off = 48 * 2.0 ** -24 * (1 + inv) * np.maximum(d, 1)
+            w0 = np.where(w > 0, w, 0)
+            den = w0.sum()
+            bound = off[w > -off].sum() + len(r) * 2.0 ** -23 * den
+            assert abs(got[i, 3] - den) <= bound, (count, i, got[i, 3], den, bound)
+            if den > 100 * bound:
+                e = (w0[:, None] * Rd[r, 6:9]).sum(0) / den
+                assert np.abs(got[i, :3] - e).max() <= 2 * bound / den + len(r) * 2.0 ** -23
+                weighted += 1
+        assert weighted > 20
+        ic.close()
+    sc.close()
+    m.close()
