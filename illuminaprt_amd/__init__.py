@@ -131,6 +131,7 @@ SIGNATURES = {
     "ilm_device_memory": (C.c_int, [_vp, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]),
     "ilm_ctx_fail_allocations": (C.c_int, [_vp, _i64, _i64]),
     "ilm_ctx_set_trace_refill": (C.c_int, [_vp, C.c_int]),
+    "ilm_ctx_get_trace_refill": (C.c_int, [_vp, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "ilm_alloc": (C.c_int, [_vp, _sz, C.POINTER(_vp)]),
     "ilm_free": (C.c_int, [_vp, _vp]),
     "ilm_upload": (C.c_int, [_vp, _vp, _vp, _sz]),
@@ -323,6 +324,12 @@ class Context:
 
     def set_trace_refill(self, idle_lanes: int):
         check(load().ilm_ctx_set_trace_refill(self.h, idle_lanes))
+
+    def trace_refill(self) -> tuple[int, int]:
+        """Idle lanes that trigger a refill: in ray queries, in a frame's launches with shadow segments."""
+        q, b = C.c_int(), C.c_int()
+        check(load().ilm_ctx_get_trace_refill(self.h, C.byref(q), C.byref(b)))
+        return q.value, b.value
 
     def fail_allocations(self, skip: int = 0, count: int = 0):
         """For tests: after `skip` device allocations, refuse the next `count`."""

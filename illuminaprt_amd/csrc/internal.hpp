@@ -33,6 +33,7 @@ constexpr int kTraceSegs = 8;           // ray segments of a traversal launch (o
 constexpr int kSegCounter0 = 64;        // first segment counter in ilm_ctx::counters
 constexpr int kSegCounterStride = 64;   // 512 bytes between segment counters
 constexpr int kSegDone = 16;            // a segment's counter of finished waves, 128 bytes after its ray counter
+constexpr int kTraceRefill = 24;        // default of ilm_ctx::trace_refill
 constexpr int kCounterWords = kSegCounter0 + kTraceSegs * kSegCounterStride;
 }  // namespace ilm
 
@@ -60,7 +61,7 @@ struct ilm_ctx {
     void* build_ws = nullptr;
     size_t build_bytes = 0;
     std::atomic<bool> build_held{false};
-    int trace_refill = 24;  // idle lanes of a wave that trigger its ray refill
+    int trace_refill = ilm::kTraceRefill;  // idle lanes of a wave that trigger its ray refill
     // device allocations still to succeed, then to be refused
     // (ilm_ctx_fail_allocations); under mu
     int64_t alloc_skip = 0, alloc_fail = 0;
@@ -145,6 +146,8 @@ ilm_mesh* scene_mesh(ilm_scene* s);
 // to accum (width*height*3 doubles, may be null only if nothing is accumulated).
 int render_paths(ilm_scene* s, const ilm_render_params& p, const PathMode& mode, double* accum,
                  ilm_render_stats* stats);
+// Idle lanes that trigger a refill in a frame's launches with shadow segments.
+int bounce_refill(const ilm_ctx* ctx);
 int trace_queue(ilm_mesh* m, const ilm_ray* rays, const unsigned long long* n_dev, int64_t capacity, ilm_hit* hits,
                 uint8_t* occ, hipStream_t stream, bool rooted = false, int refill = 0);
 // One launch over two queues: closest hits of (rays, n_dev) into hits and any

@@ -29,15 +29,16 @@ constexpr int kPtBlock = 256;
 // share of the queue) measured fastest; 2 and 4 rounds, and 8 workgroups per
 // CU whatever fits, were slower.
 constexpr int kShadeRounds = 1;
-// Idle lanes by which a bounce's launches wait longer for a refill than the
-// context's threshold: they mix closest hits with shadow segments, which end
-// early and together. Thresholds 20 / 24 / 28 / 32 / 40: 1080p frames 6.09 /
-// 6.09 / 6.06 / 6.09 / 6.13 ms, 256x256 room 1.31 / 1.28 / 1.25 / 1.25 / 1.25,
-// eight rooms 8.14 / 8.00 / 7.93 / 7.90 / 7.89 (closest hits alone are
-// fastest at 16, which the context's default of 24 is near).
-constexpr int kBounceRefill = 4;
-constexpr int kCounts = 16;
-constexpr int kAccumSlots = 4;  // shadow slots per vertex summed from one batch of loads  // the integrator's device counters (PtArgs::counts), cleared per frame
+// Idle lanes that trigger a refill in a bounce's launches while the context's
+// threshold is the default: they mix closest hits with shadow segments, which
+// end early and together. Medians of nine interleaved runs at 20 / 23 / 25 /
+// 28 / 32 / 40: 1080p frames 6.14 / 6.12 / 6.10 / 6.09 / 6.10 / 6.14 ms
+// (+-0.03), 256x256 room 1.35 / 1.33 / 1.31 / 1.28 / 1.26 / 1.25 (+-0.01),
+// eight rooms 8.14 / 8.06 / 8.00 / 7.95 / 7.92 / 7.95 (+-0.05), cache frames
+// 4.52 / 4.52 / 4.51 / 4.51 / 4.51 / 4.52 (+-0.04).
+constexpr int kBounceRefill = 28;
+constexpr int kCounts = 16;  // the integrator's device counters (PtArgs::counts), cleared per frame
+constexpr int kAccumSlots = 4;  // shadow slots per vertex summed from one batch of loads
 
 struct Material {
     f3 kd, ks;
@@ -1093,7 +1094,7 @@ int render_views(ilm_scene* s, ilm_nrc* nrc, const std::vector<ilm::View>& views
     a.rr_rule = mode ? mode->rr_rule : 0;
     a.emit0 = mode ? (mode->emit0 ? 1 : 0) : 1;
     hipStream_t st = ctx->stream;
-    const int bounce_refill = std::min(ctx->trace_refill + ilm::kBounceRefill, 64);
+    const int bounce_refill = ilm::bounce_refill(ctx);
     int ev0 = 0, ev1 = 0;
     if (cache && !s->side) {
         // the side stream of cache frames, created before the frame's timing starts
@@ -1304,6 +1305,7 @@ namespace ilm {
 
 ilm_ctx* scene_ctx(ilm_scene* s) { return s->ctx; }
 ilm_mesh* scene_mesh(ilm_scene* s) { return s->mesh; }
+int bounce_refill(const ilm_ctx* ctx) { return ctx->trace_refill == kTraceRefill ? kBounceRefill : ctx->trace_refill; }
 
 int render_paths(ilm_scene* s, const ilm_render_params& p, const PathMode& mode, double* accum,
                  ilm_render_stats* stats) {

@@ -1017,6 +1017,13 @@ int ilm_ctx_set_trace_refill(ilm_ctx* ctx, int idle_lanes) {
     return ILM_OK;
 }
 
+int ilm_ctx_get_trace_refill(ilm_ctx* ctx, int* idle_lanes, int* bounce_idle_lanes) {
+    if (!ctx) return fail(ILM_ERR_INVALID, "null ctx");
+    if (idle_lanes) *idle_lanes = ctx->trace_refill;
+    if (bounce_idle_lanes) *bounce_idle_lanes = bounce_refill(ctx);
+    return ILM_OK;
+}
+
 int ilm_trace_closest(ilm_mesh* mesh, const ilm_ray* rays, int64_t n, ilm_hit* hits, void* stream) {
     return launch_trace<false, false>(mesh, rays, n, hits, nullptr, nullptr, stream);
 }

@@ -194,8 +194,13 @@ int ilm_bvh_export(ilm_mesh* mesh, void* nodes, int32_t* tri_order);
 /* Sets how many idle lanes (1..64, default 24) a traversal wave waits for
  * before it fetches new rays for them: fewer means more refills (one atomic
  * and a divergent ray load each), more means idle lanes for longer. Applies
- * to later traversal launches of the context. No reference counterpart. */
+ * to later traversal launches of the context, but for a frame's camera rays
+ * (56). With 24, set or not, a frame's launches with shadow segments wait for
+ * 28; any other value is theirs too. No reference counterpart. */
 int ilm_ctx_set_trace_refill(ilm_ctx* ctx, int idle_lanes);
+/* The thresholds in force: of ray queries, and of a frame's launches with
+ * shadow segments. Either pointer may be NULL. */
+int ilm_ctx_get_trace_refill(ilm_ctx* ctx, int* idle_lanes, int* bounce_idle_lanes);
 
 /* Closest hit for n rays. Replaces IShape::Intersects(const Ray&,
  * DifferentialSurface&) of BVHMesh (Shape/BVHMesh.cpp:114-119,169-198) and

@@ -643,3 +643,21 @@ def test_compaction_and_camera(gpu_ctx, ilm, orc):
     want = np.nonzero(prim >= 0)[0]
     assert c == len(want)
     assert np.array_equal(ib.download(np.int32, c), want)
+
+
+def test_refill_threshold_is_the_callers(ilm):
+    """A threshold that the caller sets is that of every later launch but a
+    frame's camera rays; the default lets a frame's launches with shadow
+    segments wait for 28 idle lanes."""
+    ctx = ilm.Context(0)
+    assert ctx.trace_refill() == (24, 28)
+    for lanes in (1, 4, 23, 25, 28, 61, 64):
+        ctx.set_trace_refill(lanes)
+        assert ctx.trace_refill() == (lanes, lanes)
+    for lanes in (0, 65, -1):
+        with pytest.raises(ilm.IlmError):
+            ctx.set_trace_refill(lanes)
+    assert ctx.trace_refill() == (64, 64)
+    ctx.set_trace_refill(24)
+    assert ctx.trace_refill() == (24, 28)
+    ctx.close()
