@@ -129,6 +129,7 @@ SIGNATURES = {
     "ilm_device_count": (C.c_int, [C.POINTER(C.c_int)]),
     "ilm_device_info": (C.c_int, [_vp, C.c_char_p, C.c_int, C.POINTER(C.c_int)]),
     "ilm_device_memory": (C.c_int, [_vp, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]),
+    "ilm_ctx_trim": (C.c_int, [_vp]),
     "ilm_ctx_fail_allocations": (C.c_int, [_vp, _i64, _i64]),
     "ilm_ctx_set_trace_refill": (C.c_int, [_vp, C.c_int]),
     "ilm_ctx_get_trace_refill": (C.c_int, [_vp, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
@@ -330,6 +331,10 @@ class Context:
         q, b = C.c_int(), C.c_int()
         check(load().ilm_ctx_get_trace_refill(self.h, C.byref(q), C.byref(b)))
         return q.value, b.value
+
+    def trim(self):
+        """Gives back the scratch kept for the next device build."""
+        check(load().ilm_ctx_trim(self.h))
 
     def fail_allocations(self, skip: int = 0, count: int = 0):
         """For tests: after `skip` device allocations, refuse the next `count`."""

@@ -28,7 +28,16 @@ hipStream_t pick_stream(ilm_ctx* ctx, void* stream) {
     return stream ? (hipStream_t)stream : ctx->stream;
 }
 
-hipError_t device_malloc(ilm_ctx* ctx, void** p, size_t bytes) {
+bool release_build_ws(ilm_ctx* ctx) {
+    BuildWorkspace held(ctx, true);
+    if (!held.mine || !ctx->build_ws) return false;
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess || hipFree(ctx->build_ws) != hipSuccess) return false;
+    ctx->build_ws = nullptr;
+    ctx->build_bytes = 0;
+    return true;
+}
+
+static hipError_t try_malloc(ilm_ctx* ctx, void** p, size_t bytes) {
     *p = nullptr;
     {
         std::lock_guard<std::mutex> g(ctx->mu);
@@ -47,6 +56,12 @@ hipError_t device_malloc(ilm_ctx* ctx, void** p, size_t bytes) {
     return e;
 }
 
+hipError_t device_malloc(ilm_ctx* ctx, void** p, size_t bytes) {
+    hipError_t e = try_malloc(ctx, p, bytes);
+    if (e == hipErrorOutOfMemory && release_build_ws(ctx)) e = try_malloc(ctx, p, bytes);
+    return e;
+}
+
 int ensure_spill(ilm_ctx* ctx, size_t words) {
     if (ctx->spill_words >= words) return ILM_OK;
     if (ctx->spill) {
@@ -55,7 +70,8 @@ int ensure_spill(ilm_ctx* ctx, size_t words) {
         ctx->spill = nullptr;
         ctx->spill_words = 0;
     }
-    ILM_HIP(hipMalloc(&ctx->spill, words * sizeof(uint32_t)));
+    const hipError_t e = device_malloc(ctx, (void**)&ctx->spill, words * sizeof(uint32_t));
+    if (e != hipSuccess) return fail_hip(e, "traversal spill area");
     ctx->spill_words = words;
     ++ctx->spill_generation;
     return ILM_OK;
@@ -70,13 +86,9 @@ int ensure_build_ws(ilm_ctx* ctx, size_t bytes) {
         ctx->build_ws = nullptr;
         ctx->build_bytes = 0;
     }
-    hipError_t e = hipMalloc(&ctx->build_ws, bytes);
-    if (e != hipSuccess) {
-        ctx->build_ws = nullptr;
-        return e == hipErrorOutOfMemory
-                   ? fail(ILM_ERR_NOMEM, "device allocation of " + std::to_string(bytes) + " bytes")
-                   : fail_hip(e, "hipMalloc");
-    }
+    hipError_t e = device_malloc(ctx, &ctx->build_ws, bytes);
+    if (e == hipErrorOutOfMemory) return fail(ILM_ERR_NOMEM, "device allocation of " + std::to_string(bytes) + " bytes");
+    if (e != hipSuccess) return fail_hip(e, "hipMalloc");
     ctx->build_bytes = bytes;
     return ILM_OK;
 }
@@ -167,22 +179,18 @@ int ilm_alloc(ilm_ctx* ctx, size_t bytes, void** dev) {
     ILM_HIP(hipSetDevice(ctx->device));
     void* p = nullptr;
     hipError_t e = ilm::device_malloc(ctx, &p, bytes);
-    if (e == hipErrorOutOfMemory) {
-        // the kept build workspace makes room, unless a build uses it
-        ilm::BuildWorkspace held(ctx, true);
-        if (held.mine && ctx->build_ws) {
-            ILM_HIP(hipStreamSynchronize(ctx->stream));
-            ILM_HIP(hipFree(ctx->build_ws));
-            ctx->build_ws = nullptr;
-            ctx->build_bytes = 0;
-            e = ilm::device_malloc(ctx, &p, bytes);
-        }
-    }
     if (e == hipErrorOutOfMemory) return fail(ILM_ERR_NOMEM, "device allocation of " + std::to_string(bytes) + " bytes");
     if (e != hipSuccess) return ilm::fail_hip(e, "hipMalloc");
     std::lock_guard<std::mutex> g(ctx->mu);
     ctx->allocs.insert(p);
     *dev = p;
+    return ILM_OK;
+}
+
+int ilm_ctx_trim(ilm_ctx* ctx) {
+    if (!ctx) return fail(ILM_ERR_INVALID, "null ctx");
+    ILM_HIP(hipSetDevice(ctx->device));
+    (void)ilm::release_build_ws(ctx);
     return ILM_OK;
 }
 

@@ -56,8 +56,8 @@ struct ilm_ctx {
     uint64_t spill_generation = 0;  // counts reallocations of spill (graphs key on it)
     // scratch of the device builder, grown on demand up to kBuildKeep bytes and
     // kept for the next build; held by one building thread at a time
-    // (ilm::BuildWorkspace), given back when an allocation fails and with the
-    // context
+    // (ilm::BuildWorkspace), given back when one of the context's allocations
+    // finds the device full, by ilm_ctx_trim and with the context
     void* build_ws = nullptr;
     size_t build_bytes = 0;
     std::atomic<bool> build_held{false};
@@ -86,9 +86,6 @@ struct ilm_mesh {
 };
 
 namespace ilm {
-// hipMalloc for the context; leaves no error behind for a later
-// hipGetLastError when the device is full.
-hipError_t device_malloc(ilm_ctx* ctx, void** p, size_t bytes);
 // Ensures ctx->spill holds at least `words` 32-bit words.
 int ensure_spill(ilm_ctx* ctx, size_t words);
 // Holds ctx->build_ws for a scope, if it is wanted and no other thread does.
@@ -102,6 +99,12 @@ struct BuildWorkspace {
     BuildWorkspace(const BuildWorkspace&) = delete;
     BuildWorkspace& operator=(const BuildWorkspace&) = delete;
 };
+// Frees the build workspace; false if there is none or a build uses it.
+bool release_build_ws(ilm_ctx* ctx);
+// hipMalloc for the context. On a full device the build workspace is given
+// back, unless a build uses it, and the allocation tried again; a refusal
+// leaves no error behind for a later hipGetLastError.
+hipError_t device_malloc(ilm_ctx* ctx, void** p, size_t bytes);
 // Ensures ctx->build_ws holds at least `bytes`; the caller holds it.
 constexpr size_t kBuildKeep = size_t(1) << 30;
 int ensure_build_ws(ilm_ctx* ctx, size_t bytes);

@@ -706,7 +706,7 @@ int layout_selftest(ilm_ctx* ctx) {
     static int verified = 0;
     if (verified) return ILM_OK;
     float* d = nullptr;
-    ILM_HIP(hipMalloc(&d, 512 * sizeof(float)));
+    ILM_HIP(ilm::device_malloc(ctx, (void**)&d, 512 * sizeof(float)));
     hipLaunchKernelGGL(k_layout_probe, dim3(1), dim3(64), 0, ctx->stream, d, d + 256);
     float h[512];
     hipError_t e = hipGetLastError();

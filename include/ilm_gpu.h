@@ -84,6 +84,11 @@ int ilm_device_info(ilm_ctx* ctx, char* name, int name_len, int* cu_count);
  * used to report a workload's HBM footprint. */
 int ilm_device_memory(ilm_ctx* ctx, uint64_t* free_bytes, uint64_t* total_bytes);
 
+/* Gives back the scratch that the context keeps for the next device build
+ * (ILM_BUILDER_LBVH; up to 1 GiB), as an allocation of the context that finds
+ * the device full does by itself. Other allocators of the process cannot. */
+int ilm_ctx_trim(ilm_ctx* ctx);
+
 /* For tests of error paths: of the context's device allocations that follow,
  * `skip` go ahead, the next `count` are refused as on a full device
  * (ILM_ERR_NOMEM), and later ones go ahead. count 0 ends it. */

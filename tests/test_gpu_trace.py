@@ -661,3 +661,42 @@ def test_refill_threshold_is_the_callers(ilm):
     ctx.set_trace_refill(24)
     assert ctx.trace_refill() == (24, 28)
     ctx.close()
+
+
+@pytest.mark.parametrize("caller", ["spill", "alloc", "trim"])
+def test_kept_build_scratch_makes_room(caller, ilm):
+    """A device build's scratch stays with the context: an allocation that
+    finds the device full (the traversal's spill area, a buffer) takes it back
+    and succeeds, and so can the program. It is about 300 bytes a triangle."""
+    ctx = ilm.Context(0)
+    ntri = 400000
+    pos, idx = meshgen.random_triangles(ntri, seed=5, extent=2.0, size=0.02)
+    m = ilm.Mesh(ctx, pos, idx)
+    m.build(builder=ilm.ILM_BUILDER_LBVH)
+    rays = meshgen.rays_toward(5000, pos, seed=2)
+    rb, hb = ilm.rays_to_device(ctx, rays), ctx.buffer(len(rays) * 16)
+    before = ctx.memory()[0]
+    if caller == "trim":
+        ctx.trim()
+        ctx.trim()
+    else:
+        ctx.fail_allocations(0, 1)
+    if caller == "alloc":
+        ctx.buffer(1 << 20).free()
+    m.trace_closest(rb, len(rays), hb)
+    ctx.sync()
+    ctx.fail_allocations()
+    assert ctx.memory()[0] - before > 200 * ntri - (32 << 20)   # less the spill area
+    a = hb.download(ilm.HIT_DTYPE, len(rays))
+    m.build(builder=ilm.ILM_BUILDER_LBVH)
+    m.trace_closest(rb, len(rays), hb)
+    ctx.sync()
+    b = hb.download(ilm.HIT_DTYPE, len(rays))
+    assert (a["prim"] >= 0).mean() > 0.1 and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    ctx.fail_allocations(0, 1000)
+    with pytest.raises(ilm.IlmError):
+        ctx.buffer(1 << 20)
+    ctx.fail_allocations()
+    ctx.buffer(1 << 20).free()
+    m.close()
+    ctx.close()
