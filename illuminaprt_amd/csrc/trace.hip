@@ -624,6 +624,19 @@ static int64_t useful_blocks(int64_t n, int cu_count) {
     return (waves + kBlock / 64 - 1) / (kBlock / 64);
 }
 
+// Workgroups with a ray in every lane.
+static int64_t full_blocks(int64_t n) { return std::max<int64_t>((n + kBlock - 1) / kBlock, 1); }
+
+// The spill area of a launch. A short launch spread over the chip asks for
+// more of it than its rays need; where there is no memory for that, it takes
+// the workgroups that its rays fill.
+static int spill_for(ilm_ctx* ctx, int64_t depth, int64_t& blocks, int64_t blocks_full) {
+    const int rc = ensure_spill(ctx, (size_t)(depth * blocks * kBlock));
+    if (rc == ILM_OK || blocks <= blocks_full) return rc;
+    blocks = blocks_full;
+    return ensure_spill(ctx, (size_t)(depth * blocks * kBlock));
+}
+
 template <bool ANY, bool STATS, bool DUAL = false>
 static int launch_trace(ilm_mesh* m, const ilm_ray* rays, int64_t n, ilm_hit* hits, uint8_t* occ, int32_t* stats,
                         void* stream, const unsigned long long* n_dev = nullptr, bool rooted = false,
@@ -654,7 +667,7 @@ static int launch_trace(ilm_mesh* m, const ilm_ray* rays, int64_t n, ilm_hit* hi
     int per_cu = 0;
     ILM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, 0));
     per_cu = std::max(per_cu, 1);
-    const int64_t blocks_full = std::max<int64_t>((total + kBlock - 1) / kBlock, 1);  // with a ray in every lane
+    const int64_t blocks_full = full_blocks(total);
     int64_t blocks = std::min<int64_t>((int64_t)per_cu * ctx->cu_count, useful_blocks(total, ctx->cu_count));
     TraceArgs a;
     a.nodes = reinterpret_cast<const float4*>(m->d_nodes);
@@ -687,8 +700,9 @@ static int launch_trace(ilm_mesh* m, const ilm_ray* rays, int64_t n, ilm_hit* hi
         a.spill = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(base) + kScratchCounterBytes);
     } else {
         a.spill_depth = std::max(1, m->info.stack_need + 1);
-        int rc = ensure_spill(ctx, (size_t)a.spill_depth * (size_t)a.grid_threads);
+        int rc = spill_for(ctx, a.spill_depth, blocks, blocks_full);
         if (rc) return rc;
+        a.grid_threads = blocks * kBlock;
         a.spill = ctx->spill;
         a.counters = ctx->counters;
     }
@@ -727,7 +741,7 @@ int launch_trace_inst(ilm_ctx* ctx, const void* tlas, const void* blas, const fl
     int per_cu = 0;
     ILM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, 0));
     per_cu = std::max(per_cu, 1);
-    const int64_t blocks = std::min<int64_t>((int64_t)per_cu * ctx->cu_count, useful_blocks(n, ctx->cu_count));
+    int64_t blocks = std::min<int64_t>((int64_t)per_cu * ctx->cu_count, useful_blocks(n, ctx->cu_count));
     TraceArgs a{};
     a.nodes = reinterpret_cast<const float4*>(blas);
     a.tris = reinterpret_cast<const float4*>(tris);
@@ -735,11 +749,11 @@ int launch_trace_inst(ilm_ctx* ctx, const void* tlas, const void* blas, const fl
     a.n = n;
     a.hits = hits;
     a.occ = occ;
-    a.grid_threads = blocks * kBlock;
     a.refill_min = ctx->trace_refill;
     a.spill_depth = std::max(1, stack_need + 1);
-    int rc = ensure_spill(ctx, (size_t)a.spill_depth * (size_t)a.grid_threads);
+    int rc = spill_for(ctx, a.spill_depth, blocks, full_blocks(n));
     if (rc) return rc;
+    a.grid_threads = blocks * kBlock;
     a.spill = ctx->spill;
     a.counters = ctx->counters;
     a.total_waves = (uint32_t)(blocks * (kBlock / 64));

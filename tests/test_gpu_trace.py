@@ -700,3 +700,39 @@ def test_kept_build_scratch_makes_room(caller, ilm):
     ctx.buffer(1 << 20).free()
     m.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("instances", [False, True])
+def test_short_launch_without_memory_for_the_wide_grid(instances, ilm):
+    """A short launch spread over the chip asks for a larger spill area than
+    its rays need; refused that, it traces with as many workgroups as its rays
+    fill, to the same hits, and fails only when that is refused too."""
+    pos, idx = meshgen.icosphere(4)
+    n = 3000
+    rays = meshgen.rays_toward(n, pos, seed=8)
+    hits = []
+    for refused in (0, 1, 1000):
+        ctx = ilm.Context(0)
+        m = ilm.Mesh(ctx, pos, idx)
+        m.build()
+        rb, hb, ib = ilm.rays_to_device(ctx, rays), ctx.buffer(n * 16), ctx.buffer(n * 4)
+        table = ilm.Instances(ctx, [m]) if instances else None
+        if instances:
+            table.set([(0, None, None, None)])
+        run = (lambda: table.trace_closest(rb, n, hb, ib)) if instances else (lambda: m.trace_closest(rb, n, hb))
+        ctx.fail_allocations(0, refused)
+        if refused == 1000:
+            with pytest.raises(ilm.IlmError):
+                run()
+            ctx.fail_allocations()
+        run()
+        ctx.sync()
+        ctx.fail_allocations()
+        hits.append(hb.download(ilm.HIT_DTYPE, n))
+        if instances:
+            table.close()
+        m.close()
+        ctx.close()
+    assert (hits[0]["prim"] >= 0).mean() > 0.3
+    for h in hits[1:]:
+        assert np.array_equal(h.view(np.uint32), hits[0].view(np.uint32))
