@@ -1,7 +1,8 @@
 // GPU BVH construction: a linear BVH (Karras, "Maximizing parallelism in
 // the construction of BVHs, octrees, and k-d trees", HPG 2012) over 63-bit
-// Morton codes of triangle centroids, refitted bottom-up, then collapsed to
-// the BVH4 layout the traversal kernels read, all on the device.
+// Morton codes of triangle centroids, its boxes united from aligned runs of
+// sorted leaves, then collapsed to the BVH4 layout the traversal kernels
+// read, all on the device.
 // Replaces the host BVHMesh::Compile (Shape/BVHMesh.cpp:78-107,203-269) where
 // build time matters more than tree quality (many or large scenes).
 //

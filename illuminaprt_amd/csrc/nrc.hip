@@ -17,7 +17,7 @@
 // Layers are computed as H' = W H (features x samples), weights as A. The D
 // tiles of one layer become the next layer's B operand in place: chunk c of
 // the next layer takes D tiles 2c and 2c+1, i.e. K slot 8g+e of chunk c holds
-// feature perm(c,g,e) = 16(2c + e/4) + 4g + e%4; the packed weights use the
+// feature 16(2c + e/4) + 4g + e%4; the packed weights use the
 // same K order. The backward pass chains the same way with W^T. Weight
 // gradients dW = G H^T reduce over the samples of a workgroup in registers
 // (k_train) and over the workgroups in the optimiser (k_adam).
@@ -72,8 +72,7 @@ constexpr int kF0 = 0, kFh = 12 * 512, kF5 = kFh + 32 * 512, kFwdElems = kF5 + 2
 constexpr int kBh = 0, kB5 = 32 * 512, kBwdElems = kB5 + 4 * 256;
 static_assert(kFwdElems == kParams, "every weight appears once in the forward pack");
 
-__host__ __device__ __forceinline__ int perm(int c, int g, int e) { return 16 * (2 * c + (e >> 2)) + 4 * g + (e & 3); }
-// inverse of perm for an input feature i < 64
+// The K slot (c, g, e) of an input feature i < 64 (the inverse of the order above).
 __host__ __device__ __forceinline__ void iperm(int i, int& c, int& g, int& e) {
     int q = i >> 4, r = i & 15;
     c = q >> 1;
