@@ -736,3 +736,45 @@ def test_short_launch_without_memory_for_the_wide_grid(instances, ilm):
     assert (hits[0]["prim"] >= 0).mean() > 0.3
     for h in hits[1:]:
         assert np.array_equal(h.view(np.uint32), hits[0].view(np.uint32))
+
+
+def test_threads_building_in_one_context(ilm):
+    """Device builds of several threads in one context: one holds the kept
+    scratch, the others take their own; every tree traces to its own hits."""
+    import threading
+    ctx = ilm.Context(0)
+    ntri = (40000, 60001, 25000, 90000)
+    meshes = [meshgen.random_triangles(n, seed=n, extent=2.0, size=0.03) for n in ntri]
+    built, failed = {}, []
+
+    def build(k):
+        try:
+            for _ in range(4):
+                m = ilm.Mesh(ctx, *meshes[k])
+                m.build(builder=ilm.ILM_BUILDER_LBVH)
+                if k in built:
+                    built[k].close()
+                built[k] = m
+        except Exception as e:  # noqa: BLE001 (reported by the test's own thread)
+            failed.append(e)
+    threads = [threading.Thread(target=build, args=(k,)) for k in range(len(meshes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    for k, (pos, idx) in enumerate(meshes):
+        rays = meshgen.rays_toward(3000, pos, seed=k)
+        rb, hb = ilm.rays_to_device(ctx, rays), ctx.buffer(len(rays) * 16)
+        built[k].trace_closest(rb, len(rays), hb)
+        ctx.sync()
+        got = hb.download(ilm.HIT_DTYPE, len(rays))
+        ref = ilm.Mesh(ctx, pos, idx)
+        ref.build()
+        ref.trace_closest(rb, len(rays), hb)
+        ctx.sync()
+        want = hb.download(ilm.HIT_DTYPE, len(rays))
+        assert _compare_closest(got["prim"], got["t"], want["prim"], want["t"], f"threads {k}") >= 0.9999
+        ref.close()
+        built[k].close()
+    ctx.close()
