@@ -627,13 +627,15 @@ static int64_t useful_blocks(int64_t n, int cu_count) {
 // Workgroups with a ray in every lane.
 static int64_t full_blocks(int64_t n) { return std::max<int64_t>((n + kBlock - 1) / kBlock, 1); }
 
-// The spill area of a launch. A short launch spread over the chip asks for
-// more of it than its rays need; where there is no memory for that, it takes
-// the workgroups that its rays fill.
+// The spill area of a launch. Every launch asks for that of a short one spread
+// over the whole chip, so that the area does not grow from one short launch to
+// the next (a launch captured in a graph keeps its address); where there is no
+// memory for that, it takes the workgroups that its rays fill.
 static int spill_for(ilm_ctx* ctx, int64_t depth, int64_t& blocks, int64_t blocks_full) {
-    const int rc = ensure_spill(ctx, (size_t)(depth * blocks * kBlock));
-    if (rc == ILM_OK || blocks <= blocks_full) return rc;
-    blocks = blocks_full;
+    const int64_t wide = std::max(blocks, (int64_t)ctx->cu_count * kShortWaves / (kBlock / 64));
+    const int rc = ensure_spill(ctx, (size_t)(depth * wide * kBlock));
+    if (rc == ILM_OK || wide <= blocks_full) return rc;
+    blocks = std::min(blocks, blocks_full);
     return ensure_spill(ctx, (size_t)(depth * blocks * kBlock));
 }
 

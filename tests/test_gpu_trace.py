@@ -703,6 +703,32 @@ def test_kept_build_scratch_makes_room(caller, ilm):
 
 
 @pytest.mark.parametrize("instances", [False, True])
+def test_short_launches_share_one_spill_area(instances, ilm):
+    """Once one ray has been traced, launches of up to 256 rays for each
+    workgroup of a short launch (2 per CU) allocate nothing: a launch captured
+    in a graph keeps a valid spill area whatever short launches follow."""
+    ctx = ilm.Context(0)
+    pos, idx = meshgen.icosphere(3)
+    m = ilm.Mesh(ctx, pos, idx)
+    m.build()
+    most = 2 * ctx.cu_count * 256
+    rays = np.resize(meshgen.rays_toward(5000, pos, seed=9), (most, 8))
+    rb, hb, ib = ilm.rays_to_device(ctx, rays), ctx.buffer(most * 16), ctx.buffer(most * 4)
+    table = ilm.Instances(ctx, [m])
+    table.set([(0, None, None, None)])
+    run = (lambda n: table.trace_closest(rb, n, hb, ib)) if instances else (lambda n: m.trace_closest(rb, n, hb))
+    run(1)
+    ctx.fail_allocations(0, 1000)
+    for n in (100, 250, 257, 2000, 8 * ctx.cu_count + 1, 50000, most):
+        run(n)
+    ctx.sync()
+    ctx.fail_allocations()
+    table.close()
+    m.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("instances", [False, True])
 def test_short_launch_without_memory_for_the_wide_grid(instances, ilm):
     """A short launch spread over the chip asks for a larger spill area than
     its rays need; refused that, it traces with as many workgroups as its rays
