@@ -392,3 +392,39 @@ def test_lookups_on_both_sides_of_the_thresholds_of_the_walk(gpu_ctx, ilm, varia
         ic.close()
     sc.close()
     m.close()
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("threshold", [0.3, 1.0, 3.0])
+def test_frames_by_the_masks_equal_frames_over_whole_lists(gpu_ctx, ilm, variant, threshold):
+    """Frames go by the masks at every threshold. A cache filled by one frame
+    shows the same frame again; a second cache given the same records without
+    memory for masks shows it over the whole lists: the same image bit for bit,
+    and neither places a record, since every point is covered."""
+    from illuminaprt_amd import workloads as w
+    m, sc, pos = _room(ilm, gpu_ctx)
+    cam = w.room_camera()
+    width, height = 150, 90
+    kw = dict(cache_depth=1, error_threshold=threshold, ambient_resolution=0.01, ambient_multiplier=0.08,
+              indirect_factor=1.0, miss_radiance=(0.0, 0.0, 0.0), variant=variant, ray_depth=3)
+    acc = gpu_ctx.buffer(width * height * 24)
+    show = lambda ic: ic.render(cam, width, height, 1, acc, seed=5)
+    masked, whole = ilm.IrradianceCache(sc, **kw), ilm.IrradianceCache(sc, **kw)
+    acc.zero()
+    show(masked)
+    acc.zero()
+    again = show(masked)
+    want = acc.download(np.uint64, width * height * 3)
+    assert again["records_created"] == 0 and again["lookups"] > 0
+    lists = [len(masked.node(k)[1]) for k in range(masked.info()["nodes"])]
+    assert max(lists) > 64   # lists of more than 32 records have masks
+    gpu_ctx.fail_allocations(3, 2)   # nodes, references and records go ahead, masks do not
+    whole.insert(masked.records()[:, :10])
+    gpu_ctx.fail_allocations()
+    acc.zero()
+    stats = show(whole)
+    assert stats["records_created"] == 0
+    assert np.array_equal(acc.download(np.uint64, width * height * 3), want)
+    for x in (masked, whole, sc, m):
+        x.close()
+    acc.free()
