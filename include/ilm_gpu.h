@@ -663,7 +663,9 @@ int ilm_ic_reset(ilm_ic* ic);
  * The records stay for later frames. Synchronous. */
 int ilm_ic_render(ilm_ic* ic, const ilm_render_params* params, double* accum, ilm_ic_stats* stats);
 /* Inserts records given on the host: n x 10 floats (P, N, E, Ri); RiClamp
- * is Ri clamped to [RMin, RMax] (IrradianceCache::Insert). */
+ * is Ri clamped to [RMin, RMax] (IrradianceCache::Insert). When the device
+ * copy does not fit in memory (ILM_ERR_NOMEM, here or in a frame), the cache
+ * keeps the records and the next lookup or frame copies them again. */
 int ilm_ic_insert(ilm_ic* ic, const float* records, int64_t n);
 /* Record, octree node and node-reference counts, RMin, RMax and the root
  * cell (6 floats: lo, hi). Any pointer may be NULL. */
